@@ -47,6 +47,40 @@ def test_quantize_reference_arange_f32(pkg, orc, dev, bits):
     assert np.array_equal(sc.cpu().numpy(), rs) and np.array_equal(bi.cpu().numpy(), rb)
 
 
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_quantize_every_form(pkg, orc, dev, bits, gs, f32, offset):
+    """Every group size, width and dtype at row counts that leave a partial
+    last workgroup, from 16-byte aligned rows and from rows one element off
+    (the kernels' element-wise forms); one constant and one all-zero group."""
+    rng = np.random.default_rng(bits * 1000 + gs)
+    for rows, cols in [(1, 128), (3, 384), (37, 640)]:
+        w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
+        w[0, :gs] = 0.0
+        w[-1, -gs:] = -0.25
+        src = torch.from_numpy(w).to(dev) if f32 else _bf16(orc, w, dev)
+        buf = torch.zeros(src.numel() + offset, dtype=src.dtype, device=dev)
+        wt = buf[offset:].view(rows, cols)
+        wt.copy_(src)
+        wq, sc, bi = pkg.ops.quantize(wt, gs, bits)
+        rq, rs, rb = orc.quantize(w if f32 else _np(orc, src), gs, bits, bf16=not f32)
+        assert np.array_equal(_np(orc, wq).reshape(rq.shape), rq)
+        assert np.array_equal(_np(orc, sc), rs) and np.array_equal(_np(orc, bi), rb)
+        qb = torch.zeros(wq.numel() + offset, dtype=wq.dtype, device=dev)
+        qt = qb[offset:].view(wq.shape)
+        qt.copy_(wq)
+        for odt in (torch.bfloat16, torch.float32):
+            got = pkg.ops.dequantize(qt, sc, bi, gs, bits, out_dtype=odt)
+            code = (qt.long().unsqueeze(-1) >> torch.arange(0, 32, bits, device=dev)) & (2 ** bits - 1)
+            code = code.reshape(rows, -1, gs).double()
+            # code * scale is exact in 64 bits, so the only rounding before
+            # the output's is the 64-bit sum's (2^-29 of an f32 step)
+            want = (code * sc.double()[..., None] + bi.double()[..., None]).reshape(rows, cols)
+            assert torch.equal(got, want.float().to(odt))
+
+
 def test_quantize_full_expert_bank_bit_exact(pkg, orc, dev):
     """c2 gate_proj [128, 768, 2048] at 4 bits and a c5-sized 8-bit slice."""
     g = torch.Generator(device=dev)

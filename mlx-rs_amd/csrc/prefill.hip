@@ -102,24 +102,38 @@ __device__ __forceinline__ int div_small(int n, int d, float rd) {
   return q;
 }
 
-// x & m, opaque to the optimiser so that the byte extracts below stay
-// v_cvt_f32_ubyte{0..3} (it would otherwise fold the masks into bit-field
-// extracts plus a conversion)
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+// x & m, opaque to the optimiser (it would otherwise turn the masks and the
+// conversions below into bit-field extracts)
 __device__ __forceinline__ uint32_t and_opaque(uint32_t x, uint32_t m) {
   uint32_t r;
   asm("v_and_b32 %0, %1, %2" : "=v"(r) : "v"(x), "s"(m));
   return r;
 }
 // 8 four-bit codes of one word (little end first) -> 4 words of bf16 pairs,
-// each bf16(fmaf(code, s, b)); the even codes sit in the low nibbles.
+// each bf16(fmaf(code, s, b)).  A nibble alone in the low bits of an f16 half
+// is the f16 subnormal code * 2^-24 (code * 2^-20 four bits up), and
+// v_fma_mix_f32 multiplies it as it is by s * 2^24 (s * 2^20): the product is
+// code * s exactly, so the sum is rounded once, as fmaf(code, s, b) is (for
+// |s| < 2^104, where s * 2^24 is finite).  17 instructions a word against 23
+// with a v_cvt_f32_ubyte per code: step of c3 T=4096 509 to 502 us, c4 T=2048
+// 489 to 481, bit-identical.
 __device__ __forceinline__ void dequant4(uint32_t w, float s, float b,
                                          uint32_t* o) {
-  const uint32_t lo = and_opaque(w, 0x0F0F0F0Fu);
-  const uint32_t hi = and_opaque(w >> 4, 0x0F0F0F0Fu);
+  const float s24 = s * 0x1p24f, s20 = s * 0x1p20f;
+  const uint32_t m0 = 0x000F000Fu, m1 = 0x00F000F0u, w8 = w >> 8;
+  // codes (0, 4), (1, 5), (2, 6), (3, 7)
+  const f16x2_t c04 = __builtin_bit_cast(f16x2_t, and_opaque(w, m0));
+  const f16x2_t c15 = __builtin_bit_cast(f16x2_t, and_opaque(w, m1));
+  const f16x2_t c26 = __builtin_bit_cast(f16x2_t, and_opaque(w8, m0));
+  const f16x2_t c37 = __builtin_bit_cast(f16x2_t, and_opaque(w8, m1));
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
-    o[j] = pack_bf16(__builtin_fmaf((float)((lo >> (8 * j)) & 255u), s, b),
-                     __builtin_fmaf((float)((hi >> (8 * j)) & 255u), s, b));
+  for (int j = 0; j < 2; ++j) {
+    o[2 * j] = pack_bf16(__builtin_fmaf((float)c04[j], s24, b),
+                         __builtin_fmaf((float)c15[j], s20, b));
+    o[2 * j + 1] = pack_bf16(__builtin_fmaf((float)c26[j], s24, b),
+                             __builtin_fmaf((float)c37[j], s20, b));
+  }
 }
 // 4 eight-bit codes -> 2 words of pairs
 __device__ __forceinline__ void dequant8(uint32_t w, float s, float b,

@@ -29,6 +29,7 @@ SOURCES = [
     "dispatch.hip",
     "qgemm.hip",
     "prefill.hip",
+    "prefill_reg.hip",
     "combine.hip",
     "nn.cpp",
     "profile.cpp",

@@ -223,14 +223,19 @@ constexpr int32_t kActGeglu = 1;   // gelu_approx(g) * u  (gemma4 experts)
 // Largest input dim (K) of a projection: 8 waves x 8 groups of 64.
 constexpr int kMaxInputDims = 4096;
 // Prefill kernel M-tiles: 256 rows when the experts average at least
-// MLXR_PREFILL_TALL_ROWS rows, 128 from MLXR_PREFILL_SHORT_ROWS (and always
-// for 8-bit weights), else 64 (prefill_tile_rows).  The dispatch cuts its M-tile list with the same
-// choice; tile lists are sized for the shortest tiles.
+// MLXR_PREFILL_TALL_ROWS rows; below that 64 rows (prefill_reg.hip), and 128
+// for dense bf16 weights from MLXR_PREFILL_DENSE_ROWS rows, where there is no
+// dequantisation to keep out of LDS (c8 T=2048 step 450 us either way).
+// Measured steps, 64-row tiles against the 128-row LDS tiles they replaced:
+// c6 T=2048 312 us against 344, c3 T=1536 258 / 296, c2 T=2048 306 / 325,
+// c5 T=1024 862 / 932; against 256-row tiles: c3 T=2700 384 / 411, T=4096
+// 532 / 505.  The dispatch cuts its M-tile list with the same choice; tile
+// lists are sized for the shortest tiles.
 #ifndef MLXR_PREFILL_TALL_ROWS
 #define MLXR_PREFILL_TALL_ROWS 192
 #endif
-#ifndef MLXR_PREFILL_SHORT_ROWS
-#define MLXR_PREFILL_SHORT_ROWS 64
+#ifndef MLXR_PREFILL_DENSE_ROWS
+#define MLXR_PREFILL_DENSE_ROWS 64
 #endif
 // 1: the prefill GEMM keeps each tile's scales and biases in LDS (where they
 // fit) instead of loading them every K step
@@ -300,6 +305,20 @@ hipError_t launch_qgemm_prefill(const QGemmArgs& a, int64_t x_rows,
                                 hipStream_t s, const char* profile,
                                 const QGemmArgs* shared = nullptr,
                                 int64_t shared_rows = 0);
+
+// ------------------------------------------------------------ prefill_reg.hip
+// The 64-row tiles (weights dequantised in registers); arguments as above.
+// N-tiles per unit: until a unit has MLXR_PFR_GROUPS groups of 64 inputs,
+// while at least MLXR_PFR_MIN_UNITS units are left.
+#ifndef MLXR_PFR_GROUPS
+#define MLXR_PFR_GROUPS 32
+#endif
+#ifndef MLXR_PFR_MIN_UNITS
+#define MLXR_PFR_MIN_UNITS 2048
+#endif
+hipError_t launch_qgemm_prefill_reg(const QGemmArgs& a, int64_t x_rows, int64_t max_tiles,
+                                    hipStream_t s, const char* profile,
+                                    const QGemmArgs* shared, int64_t shared_rows);
 
 // -------------------------------------------------------------- combine.hip
 // out f32 [T, d], or bf16 when bf16 (the routing weights are then bf16

@@ -351,6 +351,50 @@ def test_gather_lhs_rows_beyond_gathered_count(pkg, orc, dev, bits):
     _close(orc.bf16_to_f32(_np(orc, got)), orc.bf16_to_f32(want), bits)
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("N,K,offset", [
+    (64, 64, 0), (192, 192, 0), (320, 512, 0), (64, 576, 0), (256, 768, 0), (320, 1088, 0),
+    (64, 1152, 0), (192, 1280, 0), (128, 2048, 0), (64, 2112, 0), (192, 2304, 0), (64, 2560, 0),
+    (320, 4096, 0), (192, 512, 1), (192, 2048, 1), (64, 2048, 4)])
+def test_gather_qmm_64_row_tiles(pkg, dev, bits, N, K, offset):
+    """The M-tiled GEMM of a few tens of rows per expert: every way its scales
+    and biases load (K's groups odd, in vectors, in one or two LDS chunks;
+    arrays `offset` elements off 16-byte alignment), partial N-tiles and last
+    lines, tiles of 1 to 64 rows and an expert of two tiles.  Scales span 2^-40
+    to 2^40.  Equal to gather_mm of the dequantised weights, and within bf16
+    of a 64-bit product."""
+    counts = [64, 1, 32, 33, 65, 31, 0, 63, 2, 17, 96, 48, 30, 34, 5, 20]
+    E, B = len(counts), sum(counts)
+    assert pkg.ops.gather_qmm_tiled(B, E) and B < 64 * E
+    g = torch.Generator(device=dev)
+    g.manual_seed(K + N + bits)
+    ids = torch.repeat_interleave(torch.arange(E, device=dev), torch.tensor(counts, device=dev))
+    ids = ids[torch.randperm(B, generator=g, device=dev)].to(torch.int32)
+    x = torch.randn((B, 1, K), generator=g, device=dev).to(torch.bfloat16)
+    wq = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, N, K * bits // 32), generator=g, device=dev,
+                       dtype=torch.int64).to(torch.int32)
+
+    def at(v):
+        buf = torch.zeros(v.numel() + offset, dtype=v.dtype, device=dev)
+        buf[offset:] = v.reshape(-1)
+        return buf[offset:].view(v.shape)
+
+    p = torch.randint(-40, 41, (E, N, 1), generator=g, device=dev).float()
+    sc = at((torch.randn((E, N, K // 64), generator=g, device=dev) * 2 ** p).to(torch.bfloat16))
+    bi = at((torch.randn((E, N, K // 64), generator=g, device=dev) * 2 ** p).to(torch.bfloat16))
+    got = pkg.ops.gather_qmm(x, wq, sc, bi, None, ids, True, 64, bits)
+    w = pkg.ops.dequantize(wq, sc, bi, 64, bits)
+    assert torch.equal(got, pkg.ops.gather_mm(x, w, None, ids))
+    xd, wd = x[:, 0].double(), w.double()
+    for e in range(E):
+        r = (ids == e).nonzero()[:, 0]
+        want = xd[r] @ wd[e].t()
+        # f32 sums of K products (K 2^-24 of the sum of their sizes, K / 64 of
+        # them added last), one bf16 rounding
+        bound = 2.0 ** -8 * want.abs() + K * 2.0 ** -24 * (xd[r].abs() @ wd[e].abs().t())
+        assert bool(((got[r, 0].double() - want).abs() <= bound).all())
+
+
 def test_gather_qmm_out_of_range_index(pkg, orc, dev):
     wq, sc, bi = _qbank(pkg, orc, 4, 64, 64, 4, dev, 3)
     x = torch.ones((3, 1, 64), dtype=torch.bfloat16, device=dev)

@@ -30,6 +30,7 @@ SOURCES = [
     "qgemm.hip",
     "prefill.hip",
     "prefill_reg.hip",
+    "prefill_tall.hip",
     "combine.hip",
     "nn.cpp",
     "profile.cpp",

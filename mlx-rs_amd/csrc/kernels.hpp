@@ -222,25 +222,21 @@ constexpr int32_t kActSwiglu = 0;  // silu(g) * u  (Qwen3.5/3.6 experts)
 constexpr int32_t kActGeglu = 1;   // gelu_approx(g) * u  (gemma4 experts)
 // Largest input dim (K) of a projection: 8 waves x 8 groups of 64.
 constexpr int kMaxInputDims = 4096;
-// Prefill kernel M-tiles: 256 rows when the experts average at least
-// MLXR_PREFILL_TALL_ROWS rows; below that 64 rows (prefill_reg.hip), and 128
-// for dense bf16 weights from MLXR_PREFILL_DENSE_ROWS rows, where there is no
-// dequantisation to keep out of LDS (c8 T=2048 step 450 us either way).
-// Measured steps, 64-row tiles against the 128-row LDS tiles they replaced:
-// c6 T=2048 312 us against 344, c3 T=1536 258 / 296, c2 T=2048 306 / 325,
-// c5 T=1024 862 / 932; against 256-row tiles: c3 T=2700 384 / 411, T=4096
-// 532 / 505.  The dispatch cuts its M-tile list with the same choice; tile
-// lists are sized for the shortest tiles.
+// Prefill kernel M-tiles.  Quantised weights: 64 rows (prefill_reg.hip) while
+// the experts average no more than that, else 128 (prefill_tall.hip); steps
+// with 64- against 128-row tiles: c6 T=2048 (64 rows an expert) 301 us / 310,
+// c5 T=1024 (64) 858 / 891, c2 T=1100 (69) 229 / 199, c2 T=1536 (96) 252 / 233,
+// c3 T=2048 (128) 310 / 289, c3 T=4096 (256) 522 / 467, c7 T=2048 (128)
+// 352 / 361.  Dense bf16 weights: 256 rows when the experts average at least
+// MLXR_PREFILL_TALL_ROWS rows, 128 from MLXR_PREFILL_DENSE_ROWS (prefill.hip:
+// nothing to keep out of LDS; c8 T=2048 450 us with either height below 256),
+// else 64.  The dispatch cuts its M-tile list with the same choice; tile lists
+// are sized for the shortest tiles.
 #ifndef MLXR_PREFILL_TALL_ROWS
 #define MLXR_PREFILL_TALL_ROWS 192
 #endif
 #ifndef MLXR_PREFILL_DENSE_ROWS
 #define MLXR_PREFILL_DENSE_ROWS 64
-#endif
-// 1: the prefill GEMM keeps each tile's scales and biases in LDS (where they
-// fit) instead of loading them every K step
-#ifndef MLXR_PREFILL_SCALES_LDS
-#define MLXR_PREFILL_SCALES_LDS 1
 #endif
 constexpr int kPrefillMinTileRows = 64;
 int prefill_tile_rows(int64_t rows, int64_t experts, int bits = 4);
@@ -319,6 +315,12 @@ hipError_t launch_qgemm_prefill(const QGemmArgs& a, int64_t x_rows,
 hipError_t launch_qgemm_prefill_reg(const QGemmArgs& a, int64_t x_rows, int64_t max_tiles,
                                     hipStream_t s, const char* profile,
                                     const QGemmArgs* shared, int64_t shared_rows);
+
+// ----------------------------------------------------------- prefill_tall.hip
+// 128-row tiles of 4- and 8-bit weights, dequantised in registers.
+hipError_t launch_qgemm_prefill_tall(const QGemmArgs& a, int64_t x_rows, int64_t max_tiles,
+                                     hipStream_t s, const char* profile,
+                                     const QGemmArgs* shared, int64_t shared_rows);
 
 // -------------------------------------------------------------- combine.hip
 // out f32 [T, d], or bf16 when bf16 (the routing weights are then bf16

@@ -21,25 +21,17 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 }
 // f rounded to bf16 (the hardware conversion: round to nearest even)
 __device__ __forceinline__ float bf16_hw(float f) { return (float)(__bf16)f; }
-// silu(g) * u with the reference's bf16 rounding points
-// (crates/mlxr-lm/src/activations.rs:187-200), the sigmoid from the
-// hardware exp2 and reciprocal (about 1 ulp each in f32; the bf16 rounding
-// that follows hides that except next to a rounding boundary)
-__device__ __forceinline__ uint16_t swiglu_fast(float g_acc, float u_acc) {
-  const float g = bf16_hw(g_acc), u = bf16_hw(u_acc);
-  const float e = __builtin_amdgcn_exp2f(-g * 1.4426950408889634f);
-  const float sg = bf16_hw(__builtin_amdgcn_rcpf(1.0f + e));
-  const float h = bf16_hw(g * sg);
-  return __builtin_bit_cast(uint16_t, (__bf16)(h * u));
-}
 // a and b rounded to bf16 by one conversion (round to nearest even), as f32
 __device__ __forceinline__ f32x2_t bf16_hw2(float a, float b) {
   const uint32_t p =
       __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));
   return f32x2_t{__uint_as_float(p << 16), __uint_as_float(p & 0xffff0000u)};
 }
-// swiglu_fast of two elements, each rounding done for both at once; the
-// results packed, the first in the low half (the same values as two calls)
+// silu(g) * u of two elements with the reference's bf16 rounding points
+// (crates/mlxr-lm/src/activations.rs:187-200), each rounding done for both at
+// once; the sigmoid from the hardware exp2 and reciprocal (about 1 ulp each in
+// f32; the bf16 rounding that follows hides that except next to a rounding
+// boundary).  The results packed, the first in the low half.
 __device__ __forceinline__ uint32_t swiglu_fast2(float g0_acc, float u0_acc, float g1_acc,
                                                  float u1_acc) {
   const f32x2_t g = bf16_hw2(g0_acc, g1_acc), u = bf16_hw2(u0_acc, u1_acc);
@@ -95,9 +87,6 @@ __device__ __forceinline__ void dequant4(uint32_t w, float s24, float s20, float
     o[2 * j + 1] = pack_bf16(__builtin_fmaf((float)c26[j], s24, b),
                              __builtin_fmaf((float)c37[j], s20, b));
   }
-}
-__device__ __forceinline__ void dequant4(uint32_t w, float s, float b, uint32_t* o) {
-  dequant4(w, s * 0x1p24f, s * 0x1p20f, b, o);
 }
 // 4 eight-bit codes -> 2 words of pairs
 __device__ __forceinline__ void dequant8(uint32_t w, float s, float b,

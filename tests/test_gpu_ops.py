@@ -351,21 +351,26 @@ def test_gather_lhs_rows_beyond_gathered_count(pkg, orc, dev, bits):
     _close(orc.bf16_to_f32(_np(orc, got)), orc.bf16_to_f32(want), bits)
 
 
+# rows of each expert: up to 64 on average (64-row tiles), and above (128)
+SHORT_COUNTS = [64, 1, 32, 33, 65, 31, 0, 63, 2, 17, 96, 48, 30, 34, 5, 20]
+TALL_COUNTS = [300, 1, 127, 128, 129, 96, 97, 65, 33, 0, 64, 200]
+
+
+@pytest.mark.parametrize("counts", [SHORT_COUNTS, TALL_COUNTS], ids=["short", "tall"])
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("N,K,offset", [
     (64, 64, 0), (192, 192, 0), (320, 512, 0), (64, 576, 0), (256, 768, 0), (320, 1088, 0),
     (64, 1152, 0), (192, 1280, 0), (128, 2048, 0), (64, 2112, 0), (192, 2304, 0), (64, 2560, 0),
     (320, 4096, 0), (192, 512, 1), (192, 2048, 1), (64, 2048, 4)])
-def test_gather_qmm_64_row_tiles(pkg, dev, bits, N, K, offset):
-    """The M-tiled GEMM of a few tens of rows per expert: every way its scales
-    and biases load (K's groups odd, in vectors, in one or two LDS chunks;
-    arrays `offset` elements off 16-byte alignment), partial N-tiles and last
-    lines, tiles of 1 to 64 rows and an expert of two tiles.  Scales span 2^-40
-    to 2^40.  Equal to gather_mm of the dequantised weights, and within bf16
-    of a 64-bit product."""
-    counts = [64, 1, 32, 33, 65, 31, 0, 63, 2, 17, 96, 48, 30, 34, 5, 20]
+def test_gather_qmm_register_tiles(pkg, dev, bits, N, K, offset, counts):
+    """The M-tiled GEMMs that dequantise in registers: every way their scales
+    and biases load (K's groups odd, in vectors, in LDS chunks; arrays
+    `offset` elements off 16-byte alignment), partial N-tiles and last lines,
+    tiles of 1 row to all of them and experts of several tiles.  Scales span
+    2^-40 to 2^40.  Equal to gather_mm of the dequantised weights, and within
+    bf16 of a 64-bit product."""
     E, B = len(counts), sum(counts)
-    assert pkg.ops.gather_qmm_tiled(B, E) and B < 64 * E
+    assert pkg.ops.gather_qmm_tiled(B, E) and (B > 64 * E) == (counts is TALL_COUNTS)
     g = torch.Generator(device=dev)
     g.manual_seed(K + N + bits)
     ids = torch.repeat_interleave(torch.arange(E, device=dev), torch.tensor(counts, device=dev))

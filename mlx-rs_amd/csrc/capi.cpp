@@ -132,7 +132,8 @@ int run_gather(const char* op, const void* x, int64_t x_batch, int64_t M,
   int32_t* status = c.take<int32_t>(1);
   int32_t* ids = c.take<int32_t>(R);
   int32_t* xrow = c.take<int32_t>(R);
-  const DispatchBuffers db = carve_dispatch(c, R, E, status);
+  DispatchBuffers db = carve_dispatch(c, R, E, status);
+  db.work_rows = work_rows_for(R, E, K, 0, bits);
   uint16_t* ob = static_cast<uint16_t*>(out);
   st = from_hip(launch_gather_prep(lhs_indices, rhs_indices, B, M, x_batch, E,
                                    N, ids, xrow, ob, status, s),
@@ -153,6 +154,7 @@ int run_gather(const char* op, const void* x, int64_t x_batch, int64_t M,
   a.num_active = db.num_active;
   a.work = db.work;
   a.num_work = db.num_work;
+  a.work_rows = db.work_rows;
   a.tiles = db.tiles;
   a.num_tiles = db.num_tiles;
   a.sorted = db.sorted;
@@ -168,7 +170,7 @@ int run_gather(const char* op, const void* x, int64_t x_batch, int64_t M,
   a.out_ld = N;
   a.out_by_flat = true;
   a.gated = false;
-  return finish(from_hip(launch_qgemm(a, R, dispatch_max_work(R, E),
+  return finish(from_hip(launch_qgemm(a, R, dispatch_max_work(R, E, db.work_rows),
                                       nn::use_prefill_path(R, E, bits), s),
                          op));
 }

@@ -144,7 +144,7 @@ __device__ __forceinline__ void dispatch_scan_body(int n, int E, int nb, int til
   // M-tiles
   const int has = (tid < E && cnt > 0) ? 1 : 0;
   int nw_long, nw_short;
-  work_counts(cnt, tid < E, nw_long, nw_short);
+  work_counts(cnt, tid < E, b.work_rows, nw_long, nw_short);
   const int nt = (tid < E) ? (cnt + tile_rows - 1) / tile_rows : 0;
   int ex[5], tot[5];
   block_exclusive_scan<5>({cnt, has, nw_long, nw_short, nt}, ex, tot, wsum);
@@ -175,10 +175,10 @@ __device__ __forceinline__ void dispatch_scan_body(int n, int E, int nb, int til
     const int* start = i < tot[2] ? s_wlong : s_wshort;
     const int e = upper_slot(start, E, i), j = i - start[e];
     const int cnt_e = (e + 1 < E ? s_off[e + 1] : total) - s_off[e];
-    int32_t* w = b.work + kWorkInts * i;
+    int32_t* w = b.work + work_ints(b.work_rows) * i;
     w[0] = e;
-    w[1] = s_off[e] + j * kWorkRows;
-    w[2] = min(kWorkRows, cnt_e - j * kWorkRows);
+    w[1] = s_off[e] + j * b.work_rows;
+    w[2] = min(b.work_rows, cnt_e - j * b.work_rows);
     w[3] = cnt_e;
   }
   for (int i = tid; i < n_tiles; i += kDispatchBlock) {
@@ -232,11 +232,13 @@ __global__ __launch_bounds__(kDispatchBlock) void dispatch_scatter_kernel(
   const int pos = base + r;
   b.sorted[pos] = (int32_t)i;
   b.inv[i] = pos;
-  b.work[kWorkInts * (b.work_first[e] + r / kWorkRows) + 4 + r % kWorkRows] =
+  const int wr = b.work_rows;  // a power of two
+  b.work[work_ints(wr) * (b.work_first[e] + r / wr) + 4 + (r & (wr - 1))] =
       (int32_t)i;
 }
 
 // n <= 1024 ids: the whole sort in one workgroup.
+template <int WR>
 __global__ __launch_bounds__(kDispatchBlock) void dispatch_small_kernel(
     const int32_t* __restrict__ ids, int n, int E, int tile_rows,
     DispatchBuffers b, int reset_status) {
@@ -244,13 +246,13 @@ __global__ __launch_bounds__(kDispatchBlock) void dispatch_small_kernel(
   if (reset_status && threadIdx.x == 0) *b.status = 0;
   __syncthreads();
   const int id = (int)threadIdx.x < n ? ids[threadIdx.x] : -1;
-  block_dispatch(id, n, E, tile_rows, b, &ls);
+  block_dispatch<WR>(id, n, E, tile_rows, b, &ls);
 }
 
 // Decode routing in one workgroup (T * K <= 1024): top-K of every token
 // (16 waves over the tokens), the renormalised weights, the status reset and
 // the counting sort of the T * K expert ids.
-template <int SLOTS, bool BF16>
+template <int SLOTS, bool BF16, int WR>
 __global__ __launch_bounds__(kDispatchBlock) void route_small_kernel(
     const float* __restrict__ logits, int64_t ld, int T, int E, int K,
     int32_t* __restrict__ idx, float* __restrict__ wts, int tile_rows,
@@ -272,7 +274,7 @@ __global__ __launch_bounds__(kDispatchBlock) void route_small_kernel(
   }
   __syncthreads();
   const int n = T * K;
-  block_dispatch((int)threadIdx.x < n ? ids[threadIdx.x] : -1, n, E,
+  block_dispatch<WR>((int)threadIdx.x < n ? ids[threadIdx.x] : -1, n, E,
                  tile_rows, b, &ls);
 }
 
@@ -321,7 +323,7 @@ __global__ __launch_bounds__(kDispatchBlock) void route_wave_kernel(
 // or acquire fence: on this part those write back and invalidate the whole
 // L2.  *counter is 0 when the launch starts (the logits launch before it
 // clears it); the status word is cleared and set by the last workgroup only.
-template <int SLOTS, bool BF16>
+template <int SLOTS, bool BF16, int WR>
 __global__ __launch_bounds__(kDispatchBlock) void route_fused_kernel(
     const float* __restrict__ logits, int64_t ld, int T, int E, int K,
     int32_t* idx, float* __restrict__ wts, int tile_rows, DispatchBuffers b,
@@ -354,7 +356,7 @@ __global__ __launch_bounds__(kDispatchBlock) void route_fused_kernel(
                      ? __hip_atomic_load(idx + threadIdx.x, __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT)
                      : -1;
-  block_dispatch(id, n, E, tile_rows, b, &ls);
+  block_dispatch<WR>(id, n, E, tile_rows, b, &ls);
 }
 
 __global__ __launch_bounds__(256) void dispatch_identity_kernel(
@@ -367,7 +369,7 @@ __global__ __launch_bounds__(256) void dispatch_identity_kernel(
     b.offsets[1] = n;
     b.active[0] = 0;
     *b.num_active = n > 0 ? 1 : 0;
-    *b.num_work = (n + kWorkRows - 1) / kWorkRows;
+    *b.num_work = (n + b.work_rows - 1) / b.work_rows;
     *b.num_tiles = n_tiles;
   }
   for (int j = tid; j < n_tiles; j += 256) {
@@ -378,13 +380,13 @@ __global__ __launch_bounds__(256) void dispatch_identity_kernel(
     b.sorted[i] = i;
     b.inv[i] = i;
   }
-  for (int j = tid; j * kWorkRows < n; j += 256) {
-    int32_t* w = b.work + kWorkInts * j;
+  for (int j = tid; j * b.work_rows < n; j += 256) {
+    int32_t* w = b.work + work_ints(b.work_rows) * j;
     w[0] = 0;
-    w[1] = j * kWorkRows;
-    w[2] = min(kWorkRows, n - j * kWorkRows);
+    w[1] = j * b.work_rows;
+    w[2] = min(b.work_rows, n - j * b.work_rows);
     w[3] = n;
-    for (int i = 0; i < kWorkRows; ++i) w[4 + i] = j * kWorkRows + i;
+    for (int i = 0; i < b.work_rows; ++i) w[4 + i] = j * b.work_rows + i;
   }
 }
 
@@ -430,8 +432,12 @@ hipError_t launch_dispatch(const int32_t* ids, int64_t n, int64_t E,
                            bool reset_status, hipStream_t s, int32_t* counter) {
   ProfileScope prof("dispatch", s);
   if (n <= kDispatchBlock) {
-    dispatch_small_kernel<<<1, kDispatchBlock, 0, s>>>(
-        ids, (int)n, (int)E, tile_rows, b, reset_status ? 1 : 0);
+    if (b.work_rows == kWorkRowsWide)
+      dispatch_small_kernel<kWorkRowsWide><<<1, kDispatchBlock, 0, s>>>(
+          ids, (int)n, (int)E, tile_rows, b, reset_status ? 1 : 0);
+    else
+      dispatch_small_kernel<kWorkRows><<<1, kDispatchBlock, 0, s>>>(
+          ids, (int)n, (int)E, tile_rows, b, reset_status ? 1 : 0);
     return hipGetLastError();
   }
   const int nb = (int)((n + kDispatchBlock - 1) / kDispatchBlock);
@@ -463,8 +469,11 @@ void route_small_launch(const float* logits, int64_t ld, int64_t T, int64_t E,
     if (one_wave)                                                          \
       route_wave_kernel<S, BF16><<<1, threads, 0, s>>>(                    \
           logits, ld, (int)T, (int)E, (int)K, idx, wts, tile_rows, b);     \
+    else if (b.work_rows == kWorkRowsWide)                                 \
+      route_small_kernel<S, BF16, kWorkRowsWide><<<1, kDispatchBlock, 0, s>>>( \
+          logits, ld, (int)T, (int)E, (int)K, idx, wts, tile_rows, b);     \
     else                                                                   \
-      route_small_kernel<S, BF16><<<1, kDispatchBlock, 0, s>>>(            \
+      route_small_kernel<S, BF16, kWorkRows><<<1, kDispatchBlock, 0, s>>>( \
           logits, ld, (int)T, (int)E, (int)K, idx, wts, tile_rows, b);     \
   } while (0)
   if (slots <= 1)
@@ -487,8 +496,14 @@ void route_fused_launch(const float* logits, int64_t ld, int64_t T, int64_t E,
   const int slots = (int)((E + 63) / 64);
   const unsigned grid = (unsigned)((T + MLXR_ROUTE_FUSED_TPW - 1) / MLXR_ROUTE_FUSED_TPW);
 #define MLXR_RF(S)                                                                 \
-  route_fused_kernel<S, BF16><<<grid, kDispatchBlock, 0, s>>>(                     \
-      logits, ld, (int)T, (int)E, (int)K, idx, wts, tile_rows, b, counter)
+  do {                                                                             \
+    if (b.work_rows == kWorkRowsWide)                                              \
+      route_fused_kernel<S, BF16, kWorkRowsWide><<<grid, kDispatchBlock, 0, s>>>(  \
+          logits, ld, (int)T, (int)E, (int)K, idx, wts, tile_rows, b, counter);    \
+    else                                                                           \
+      route_fused_kernel<S, BF16, kWorkRows><<<grid, kDispatchBlock, 0, s>>>(      \
+          logits, ld, (int)T, (int)E, (int)K, idx, wts, tile_rows, b, counter);    \
+  } while (0)
   if (slots <= 1)
     MLXR_RF(1);
   else if (slots <= 2)

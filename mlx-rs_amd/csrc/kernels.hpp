@@ -110,8 +110,8 @@ struct DispatchBuffers {
   int32_t* inv;         // [n]  sorted slot per flat index
   int32_t* active;      // [E]  experts with rows, ascending
   int32_t* num_active;  // [1]
-  int32_t* work;        // [max_work][kWorkInts] work item records: each
-                        // expert's rows in chunks of at most kWorkRows
+  int32_t* work;        // work item records: each expert's rows in chunks of
+                        // at most work_rows
   int32_t* num_work;    // [1]
   int32_t* work_first;  // [E] first work item of each expert
   int32_t* tiles;       // [max_tiles] packed (expert, first row) of M-tiles
@@ -119,17 +119,21 @@ struct DispatchBuffers {
   int32_t* block_hist;  // [ceil(n/1024), E] scratch
   int32_t* rank;        // [n] scratch
   int32_t* status;      // [1] 0 ok, 1 id out of range
+  int32_t work_rows;    // rows per work item: kWorkRows or kWorkRowsWide
 };
 constexpr int kDispatchBlock = 1024;
 constexpr int kMaxExperts = 1024;
 // Rows per decode work item: an expert with more rows becomes several items,
 // so the decode GEMM's work items stay small and alike.
 constexpr int kWorkRows = 8;
-// Work item record: expert, first sorted slot, rows (<= kWorkRows), rows of
+// ... and of the wide items (work_rows_for), where experts of more rows are
+// common: the weights are then read once per 16 rows.
+constexpr int kWorkRowsWide = 16;
+// Work item record: expert, first sorted slot, rows (<= work_rows), rows of
 // the whole expert, then the flat row index (sorted[slot]) of each of the
 // item's slots (unset past rows).  A GEMM workgroup learns its task, and
 // where its x rows live, from these 48 bytes without a dependent load.
-constexpr int kWorkInts = 4 + kWorkRows;
+__host__ __device__ constexpr int work_ints(int work_rows) { return 4 + work_rows; }
 // The streaming decode GEMM runs the items of experts with at most this many
 // rows in its 4-token MFMA form, the others in the 8-token form (longer per
 // item: the dispatch lists their items first, so the long workgroups start
@@ -140,8 +144,26 @@ constexpr int kWorkInts = 4 + kWorkRows;
 constexpr int kStreamTT4Rows = MLXR_STREAM_TT4_ROWS;
 int64_t dispatch_max_tiles(int64_t n, int64_t E, int tile_rows);
 // Bound on the work items of n flat rows over E experts.
-inline int64_t dispatch_max_work(int64_t n, int64_t E) {
-  return (E < n ? E : n) + n / kWorkRows;
+inline int64_t dispatch_max_work(int64_t n, int64_t E, int work_rows = kWorkRows) {
+  return (E < n ? E : n) + n / work_rows;
+}
+// Rows per work item of a call whose GEMMs have input dims K0 and K1 (0: one
+// GEMM): wide items from MLXR_WIDE_ITEM_ROWS rows per expert, where more than
+// one in seven experts has over kWorkRows rows: at 6 rows per expert a step of
+// c2 (T = 96) went from 117 us to 114, c6 (T = 200) 193 to 188; with fewer, the
+// 8-row items' kernel covers nearly every expert in one item and has the
+// smaller LDS and register footprint.  For quantised weights and
+// input dims that the wide form stages (stream16_body); more than 64 rows (the
+// one-wave sort of fewer makes 8-row items).
+#ifndef MLXR_WIDE_ITEM_ROWS
+#define MLXR_WIDE_ITEM_ROWS 6
+#endif
+constexpr int kWideWhole = 1536, kWideSlice = 1024;
+inline int work_rows_for(int64_t n, int64_t E, int64_t K0, int64_t K1, int bits) {
+  const auto fits = [](int64_t k) { return k <= kWideWhole || k % kWideSlice == 0; };
+  return bits != 16 && n > 64 && n >= MLXR_WIDE_ITEM_ROWS * E && fits(K0) && fits(K1)
+             ? kWorkRowsWide
+             : kWorkRows;
 }
 // Clears a workspace status word with a one-thread kernel (no memset node,
 // so the call stays valid under stream capture).
@@ -198,10 +220,11 @@ struct QGemmArgs {
   const int32_t* row_map;
   int32_t row_div;
   bool x_by_slot;
+  uint8_t work_rows;       // rows per work item (in what would be padding)
   const int32_t* offsets;  // [E+1] slot range of each expert
   const int32_t* active;   // [E] experts with rows
   const int32_t* num_active;
-  const int32_t* work;     // work item records (kWorkInts each)
+  const int32_t* work;     // work item records (work_ints(work_rows) each)
   const int32_t* num_work;
   const int32_t* tiles;    // M-tile list (prefill path)
   const int32_t* num_tiles;

@@ -68,7 +68,11 @@ DispatchBuffers carve_dispatch(Carve& c, int64_t n, int64_t E,
   b.inv = c.take<int32_t>(n);
   b.active = c.take<int32_t>(E);
   b.num_active = c.take<int32_t>(1);
-  b.work = c.take<int32_t>(kWorkInts * dispatch_max_work(n, E));
+  // (room for the items of either size)
+  b.work = c.take<int32_t>(
+      std::max(work_ints(kWorkRows) * dispatch_max_work(n, E, kWorkRows),
+               work_ints(kWorkRowsWide) * dispatch_max_work(n, E, kWorkRowsWide)));
+  b.work_rows = kWorkRows;
   b.num_work = c.take<int32_t>(1);
   b.work_first = c.take<int32_t>(E);
   b.tiles = c.take<int32_t>(2 * dispatch_max_tiles(n, E, kPrefillMinTileRows));
@@ -83,7 +87,7 @@ namespace nn {
 
 bool use_prefill_path(int64_t rows, int64_t experts, int bits) {
   // Dense bf16 weights: the split-K kernel reads an expert's weights once
-  // per work item (kWorkRows rows), the M-tiled one once per M-tile, with
+  // per work item (of 8 or 16 rows), the M-tiled one once per M-tile, with
   // no dequantisation to pay for; it takes over from
   // MLXR_DENSE_TILED_ROWS rows per expert (measured on the c8 block: 2),
   // given rows enough for its tiles to fill the GPU (one expert with 16
@@ -135,7 +139,8 @@ void SwigluMlp::plan(Carve& ws, int64_t T, int64_t d, int64_t f) {
 Status SwigluMlp::forward(const uint16_t* x, int64_t T, uint16_t* y,
                           Carve& ws, int32_t* status, hipStream_t s) const {
   const int64_t d = gate_.input_dims, f = gate_.output_dims;
-  const DispatchBuffers db = carve_dispatch(ws, T, 1, status);
+  DispatchBuffers db = carve_dispatch(ws, T, 1, status);
+  db.work_rows = work_rows_for(T, 1, d, f, gate_.bits);
   uint16_t* act = ws.take<uint16_t>(T * f);
   Status st = from_hip(launch_dispatch_identity(T, prefill_tile_rows(T, 1, gate_.bits), db, s),
                        "shared_expert dispatch");
@@ -154,6 +159,7 @@ Status SwigluMlp::forward(const uint16_t* x, int64_t T, uint16_t* y,
   g.num_active = db.num_active;
   g.work = db.work;
   g.num_work = db.num_work;
+  g.work_rows = db.work_rows;
   g.tiles = db.tiles;
   g.num_tiles = db.num_tiles;
   g.sorted = db.sorted;
@@ -168,7 +174,7 @@ Status SwigluMlp::forward(const uint16_t* x, int64_t T, uint16_t* y,
   g.out = act;
   g.out_ld = f;
   g.gated = true;
-  const int64_t items = dispatch_max_work(T, 1);
+  const int64_t items = dispatch_max_work(T, 1, db.work_rows);
   st = from_hip(launch_qgemm(g, T, items, prefill, s, "shared_gated"),
                 "shared_expert gate/up");
   if (!st.ok) return st;
@@ -286,7 +292,8 @@ Status SwitchFfn::forward(const uint16_t* x, int64_t T, const int32_t* indices,
   if (combined) *combined = false;
   const int64_t E = sw_.E;
   const int64_t n = T * K;
-  const DispatchBuffers db = carve_dispatch(ws, n, E, status);
+  DispatchBuffers db = carve_dispatch(ws, n, E, status);
+  db.work_rows = work_rows_for(n, E, sw_.d, sw_.f, sw_.bits);
   // (the dispatch clears *status first: no launch of its own for that)
   Status st = from_hip(
       launch_dispatch(indices, n, E, prefill_tile_rows(n, E, sw_.bits), db, true, s),
@@ -318,7 +325,7 @@ Status SwitchFfn::experts(const uint16_t* x, int64_t T, int64_t K,
   const int64_t d = sw_.d, f = sw_.f, E = sw_.E;
   const int64_t n = T * K;
   uint16_t* act = ws.take<uint16_t>(n * f);
-  const int64_t max_items = dispatch_max_work(n, E);
+  const int64_t max_items = dispatch_max_work(n, E, db.work_rows);
   const bool prefill = use_prefill_path(n, E, sw_.bits);
   QGemmArgs g{};
   g.x = x;
@@ -333,6 +340,7 @@ Status SwitchFfn::experts(const uint16_t* x, int64_t T, int64_t K,
   g.num_active = db.num_active;
   g.work = db.work;
   g.num_work = db.num_work;
+  g.work_rows = db.work_rows;
   g.tiles = db.tiles;
   g.num_tiles = db.num_tiles;
   g.sorted = db.sorted;
@@ -508,7 +516,9 @@ Status Qwen35MoeBlock::forward(const uint16_t* x, int64_t T, void* out,
   Carve shared_ws = ws;  // the shared expert's scratch (plan order)
   if (shared) SwigluMlp::plan(ws, T, d, b_.shared_expert_intermediate_size);
   uint16_t* y = ws.take<uint16_t>(T * K * d);
-  const DispatchBuffers db = carve_dispatch(ws, T * K, E, status);
+  DispatchBuffers db = carve_dispatch(ws, T * K, E, status);
+  db.work_rows =
+      work_rows_for(T * K, E, d, b_.moe_intermediate_size, b_.switch_mlp.gate_proj.bits);
   // gate.forward + shared_expert_gate.forward (moe.rs:118,123) in one pass.
   RouterWeights rw = router_weights_f32(
       b_.gate_weight, shared ? b_.shared_expert_gate_weight : nullptr);

@@ -292,10 +292,11 @@ __device__ __forceinline__ void decode_body(const QGemmArgs& a, int tile,
     int64_t xrow = 0;
     if (tv) {
       const int slot = row0 + tok;
-      // this lane's flat row from the record (tok < kWorkRows = 8)
+      // this lane's flat row from the record (its first eight fetched with the
+      // header)
       const int f4 = (tok & 3) == 0 ? fr0.x : (tok & 3) == 1 ? fr0.y : (tok & 3) == 2 ? fr0.z : fr0.w;
       const int f8 = (tok & 3) == 0 ? fr1.x : (tok & 3) == 1 ? fr1.y : (tok & 3) == 2 ? fr1.z : fr1.w;
-      const int flat = tok < 4 ? f4 : f8;
+      const int flat = tok < 4 ? f4 : tok < 8 ? f8 : a.x_by_slot ? 0 : rec[4 + tok];
       xrow = a.x_by_slot ? slot : (a.row_map ? a.row_map[flat] : flat / a.row_div);
     }
     f32x4_t acc[CB][NM];
@@ -445,15 +446,17 @@ __device__ __forceinline__ void decode_body(const QGemmArgs& a, int tile,
 // The unit of workgroup blockIdx.x: a work item of the routed problem `a`
 // (its record, fetched whole: header and flat rows), or, from units1 on,
 // an item of a folded second problem -- the block's shared expert, every
-// token's row once: item i is rows 8i..8i+7 of `rows2` in token order, its
-// record made here (expert 0, the rows' own slots, no dispatch).  Returns
-// false for an idle workgroup (past the routed problem's items).
+// token's row once: item i is rows 8i..8i+7 (16i..16i+15 of wide items) of
+// `rows2` in token order, its record made here (expert 0, the rows' own slots,
+// no dispatch).  Returns false for an idle workgroup (past the routed problem's
+// items).
 struct Unit {
   const int32_t* rec;
   int4 wk, fr0, fr1;
   int tile;
   bool shared;
 };
+template <int WR = 0>  // rows per item, or 0: a.work_rows
 __device__ __forceinline__ bool decode_unit(const QGemmArgs& a, int tiles_n,
                                             int units1, int items1, int rows2,
                                             Unit& u) {
@@ -463,14 +466,15 @@ __device__ __forceinline__ bool decode_unit(const QGemmArgs& a, int tiles_n,
   u.tile = v - ai * tiles_n;
   // (the routed record is read unconditionally, item 0's for a shared
   // unit)
-  u.rec = a.work + (int64_t)kWorkInts * (u.shared ? 0 : min(ai, items1 - 1));
+  const int wr = WR ? WR : a.work_rows;
+  u.rec = a.work + (int64_t)work_ints(wr) * (u.shared ? 0 : min(ai, items1 - 1));
   u.wk = *reinterpret_cast<const int4*>(u.rec);
   u.fr0 = *reinterpret_cast<const int4*>(u.rec + 4);
   u.fr1 = *reinterpret_cast<const int4*>(u.rec + 8);
   const int n_act = *a.num_work;
   if (u.shared) {
-    const int r0 = kWorkRows * ai;
-    u.wk = make_int4(0, r0, min(kWorkRows, rows2 - r0), rows2);
+    const int r0 = wr * ai;
+    u.wk = make_int4(0, r0, min(wr, rows2 - r0), rows2);
     u.fr0 = make_int4(r0, r0 + 1, r0 + 2, r0 + 3);
     u.fr1 = make_int4(r0 + 4, r0 + 5, r0 + 6, r0 + 7);
     return true;
@@ -518,7 +522,6 @@ __device__ __forceinline__ void stream_body(const QGemmArgs& a,
                                             char* smem, int ltid, int lthreads,
                                             uint16_t* yl, int yrow_off) {
   constexpr int nb = NB;
-  static_assert(kWorkRows <= 8, "an item of a >4-row expert fits TT = 8");
   constexpr int NM = GATED ? 2 : 1;
   constexpr int NA = 2 * NM;            // scale and bias arrays
   constexpr int GG = 16 / TT;           // groups per MFMA
@@ -531,7 +534,8 @@ __device__ __forceinline__ void stream_body(const QGemmArgs& a,
   // grids: more, shorter waves); their sums meet in LDS at the end
   const int waves = (lthreads >> 6) / KS;  // channel waves
   // items of experts with at most 4 rows run with TT = 4, the others with
-  // TT = 8 >= kWorkRows: an item is always one pass
+  // TT = 8 (wide items of more than 8 rows in stream16_body): an item is
+  // always one pass
   const int e = wk.x, row0 = wk.y, nt = min(wk.z, TT);
   const int lane = ltid & 63, wave_id = ltid >> 6;
   const int wave = wave_id / KS, kq = wave_id % KS;  // channel wave, K-slice
@@ -844,6 +848,271 @@ __device__ __forceinline__ void stream_body(const QGemmArgs& a,
   }
 }
 
+// The wide form: an item of 9 to 16 rows (of an expert of more than 8), so
+// that an expert's weights are read once per 16 rows where the 8-token form
+// reads them per 8.  A wave loads the same bytes per super-step (two groups of
+// its 16 channels) as there; the MFMA's 16 A rows are 16 tokens, so all lanes
+// must hold one group's codes: v_permlane32_swap_b32 turns two words of a
+// lane, of group A on lanes 0-31 and B on 32-63, into a word of A and one of B
+// on every lane.  Lane quarter q then supplies codes 16 i + 32 (q & 1) +
+// 8 (q >> 1) .. + 7 of the group to MFMA i of two, and receives tokens
+// 4 q .. 4 q + 3 of channel l % 16: no sums cross lanes.  x is staged whole up
+// to kWideWhole inputs, else kWideSlice at a time (so that three workgroups
+// still share a CU), NB = 1 then.
+// 12 rows an expert of c7 (T = 190): gate/up 83 us in 8-row items, 72 in these,
+// down 59 and 44.  Steps of c2 at 8, 10 and 14 rows an expert (T = 128, 160,
+// 224): 128, 151, 186 us and 117, 130, 154; c5 at 6 (T = 200) 893 and 810.
+template <int BITS, bool GATED, int NB>
+__device__ __forceinline__ void stream16_body(const QGemmArgs& a, const int32_t* rec, int4 wk,
+                                              int tile, char* smem) {
+  constexpr int TT = 16, D = 3, R = D + 1;
+  constexpr int NM = GATED ? 2 : 1, NA = 2 * NM;
+  constexpr int NL = BITS / 4;     // 16-byte loads per lane and super-step
+  constexpr int WPG = 2 * BITS;    // packed words per row and group
+  const int e = wk.x, row0 = wk.y, nt = min(wk.z, TT);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n = lane & 15, q = lane >> 4;
+  const int K = a.K, groups = K >> 6, ssteps = groups >> 1;
+  const int KS = K <= kWideWhole ? K : kWideSlice;  // inputs of x staged at once
+  const int slices = K / KS, sps = ssteps / slices;  // super-steps per slice
+  const int total = NB * ssteps;
+  // LDS as stream_body: x [16][KS + 8], X [KS / 64][16], the waves' scales
+  const int xs = KS + 8;
+  uint16_t* xl = reinterpret_cast<uint16_t*>(smem);
+  float* Xl = reinterpret_cast<float*>(smem + (size_t)TT * xs * 2);
+  char* sb_base = smem + (size_t)TT * xs * 2 + (size_t)(KS >> 6) * TT * 4;
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  const u32x4_t zq = {0u, 0u, 0u, 0u};
+  const int ch0 = ((tile * MLXR_STREAM_WAVES + wave) * NB) * 16 + n;
+  const int64_t wrow0 = (int64_t)e * a.e_rows + ch0;
+
+  struct Ring {
+    u32x4_t w[NM][NL];
+  };
+  const uint32_t* wb[NM];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    const QWeights& W = m == 0 ? a.w0 : a.w1;
+    wb[m] = W.w + (wrow0 * groups + (q >> 1)) * WPG + (q & 1) * BITS;
+  }
+  const int64_t blk_rows = (int64_t)16 * groups;
+  auto load = [&](Ring& r, int gs) {
+    const int bi = gs / ssteps, ss = gs - bi * ssteps;
+    const int64_t go = bi * blk_rows + 2 * ss;
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+      const u32x4_t* wp = reinterpret_cast<const u32x4_t*>(wb[m] + go * WPG);
+#pragma unroll
+      for (int i = 0; i < NL; ++i) r.w[m][i] = wp[i];
+    }
+  };
+  // x: thread -> 16-byte chunks tid % 128, + 128, .. of rows 8 (tid / 128) + t
+  const int k8 = tid & 127, rh = 8 * (tid >> 7), rows_h = nt - rh;
+  int64_t xr[8];
+  {
+    const int4 f0 = *reinterpret_cast<const int4*>(rec + 4 + rh);
+    const int4 f1 = *reinterpret_cast<const int4*>(rec + 8 + rh);
+    const int fl[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+    int32_t rm[8];
+    if (!a.x_by_slot && a.row_map) {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) rm[t] = a.row_map[t < rows_h ? fl[t] : rec[4]];
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      int64_t r = 0;
+      if (t < rows_h)
+        r = a.x_by_slot ? row0 + rh + t : (a.row_map ? rm[t] : fl[t] / a.row_div);
+      xr[t] = r;
+    }
+  }
+  const int per_row = KS >> 3;
+  auto load_x = [&](int k, u32x4_t (&v)[8]) {  // chunk k of all of K's
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      v[t] = zq;
+      if (t < rows_h) v[t] = *reinterpret_cast<const u32x4_t*>(a.x + xr[t] * a.x_ld + 8 * k);
+    }
+  };
+  auto stage_x = [&](int kl, const u32x4_t (&v)[8]) {  // ... chunk kl of the slice
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      float sx = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        sx += __uint_as_float(v[t][j] << 16) + __uint_as_float(v[t][j] & 0xffff0000u);
+      sx += __shfl_xor(sx, 1, 64);
+      sx += __shfl_xor(sx, 2, 64);
+      sx += __shfl_xor(sx, 4, 64);
+      if ((kl & 7) == 0) Xl[(kl >> 3) * TT + rh + t] = sx;
+      u32x4_t w = v[t];
+      if constexpr (BITS == 4) w = perm4(w);
+      *reinterpret_cast<u32x4_t*>(xl + (size_t)(rh + t) * xs + 8 * kl) = w;
+    }
+  };
+  // issue order as stream_body: x, scales and biases, weights
+  u32x4_t xv[8];
+  load_x(min(k8, per_row - 1), xv);
+  MLXR_SCHED_BARRIER();
+  const int sbn = NB * 16 * groups, sbv = sbn >> 3;
+  uint16_t* sbl = reinterpret_cast<uint16_t*>(sb_base) + (size_t)wave * NA * sbn;
+  const uint16_t* sbsrc[NA];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    const QWeights& W = m == 0 ? a.w0 : a.w1;
+    sbsrc[2 * m] = W.scales + (wrow0 - n) * groups;
+    sbsrc[2 * m + 1] = W.biases + (wrow0 - n) * groups;
+  }
+  u32x4_t sv[NA];
+  const int sl = min(lane, sbv - 1);
+#pragma unroll
+  for (int i = 0; i < NA; ++i) sv[i] = *reinterpret_cast<const u32x4_t*>(sbsrc[i] + 8 * sl);
+  MLXR_SCHED_BARRIER();
+  Ring ring[R];
+#pragma unroll
+  for (int j = 0; j < D; ++j) load(ring[j], min(j, total - 1));
+  MLXR_SCHED_BARRIER();
+  if (k8 < per_row) stage_x(k8, xv);  // per_row is a multiple of 8: whole octets
+  for (int c8 = k8 + 128; c8 < per_row; c8 += 128) {
+    u32x4_t v[8];
+    load_x(c8, v);
+    stage_x(c8, v);
+  }
+  __syncthreads();
+  if (lane < sbv) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+      *reinterpret_cast<u32x4_t*>(sbl + i * sbn + 8 * lane) = sv[i];
+  }
+  for (int i = lane + 64; i < sbv; i += 64) {
+#pragma unroll
+    for (int j = 0; j < NA; ++j)
+      *reinterpret_cast<u32x4_t*>(sbl + j * sbn + 8 * i) =
+          *reinterpret_cast<const u32x4_t*>(sbsrc[j] + 8 * i);
+  }
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+  constexpr int ND = NB > 1 ? NB - 1 : 1;
+  f32x4_t acc[NM], done[ND][NM];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    acc[m] = zero;
+#pragma unroll
+    for (int b = 0; b < ND; ++b) done[b][m] = zero;
+  }
+  const uint32_t one_v = 0x3F803F80u;
+  const char* xsrc = smem + ((size_t)n * xs + 32 * (q & 1) + 8 * (q >> 1)) * 2;
+  for (int s = 0; s < slices; ++s) {
+    if (s > 0) {
+      // the next slice of x (kWideSlice inputs: one chunk per thread)
+      u32x4_t v[8];
+      load_x(s * per_row + k8, v);
+      __syncthreads();
+      stage_x(k8, v);
+      __syncthreads();
+    }
+    const int end = slices == 1 ? total : (s + 1) * sps;
+    for (int gs0 = s * sps; gs0 < end; gs0 += R) {
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        const int gs = gs0 + j;
+        load(ring[(j + D) % R], min(gs + D, total - 1));
+        MLXR_SCHED_BARRIER();
+        if (gs >= end) continue;  // (uniform; the loads above run on)
+        const int bi = gs / ssteps, ss = gs - bi * ssteps;
+        uint32_t w[NM][4 * NL];
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+#pragma unroll
+          for (int i = 0; i < 4 * NL; ++i) w[m][i] = ring[j].w[m][i / 4][i % 4];
+          // pairs of words (4-bit) or of word pairs (8-bit)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int h = 0; h < NL; ++h) {
+              uint32_t &lo = w[m][2 * NL * i + h], &hi = w[m][2 * NL * i + NL + h];
+              const auto r = __builtin_amdgcn_permlane32_swap(lo, hi, false, false);
+              lo = r[0];
+              hi = r[1];
+            }
+        }
+#pragma unroll
+        for (int g2 = 0; g2 < 2; ++g2) {
+          const int g = 2 * ss + g2, gl = g - s * (KS >> 6);
+          bf16x8_t xa[2];
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            xa[i] = as_bf16x8(
+                *reinterpret_cast<const u32x4_t*>(xsrc + (size_t)(64 * gl + 16 * i) * 2));
+          const f32x4_t X = *reinterpret_cast<const f32x4_t*>(Xl + gl * TT + 4 * q);
+#pragma unroll
+          for (int m = 0; m < NM; ++m) {
+            f32x4_t P = zero;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+              const int b = 2 * NL * i + NL * g2;
+              u32x4_t u;
+              if constexpr (BITS == 4)
+                u = unpack4(w[m][b], one_v);
+              else
+                u = unpack8(w[m][b], w[m][b + NL - 1]);
+              P = mfma16x16x32(xa[i], as_bf16x8(u), P);
+            }
+            const int si = (bi * 16 + n) * groups + g;
+            float sc, cb;
+            group_terms<BITS>(sbl[(m * 2) * sbn + si], sbl[(m * 2 + 1) * sbn + si], sc, cb);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              acc[m][r] = __builtin_fmaf(sc, P[r], __builtin_fmaf(cb, X[r], acc[m][r]));
+          }
+        }
+        if constexpr (NB > 1) {
+          const bool last = ss == ssteps - 1 && bi < NB - 1;
+#pragma unroll
+          for (int b = 0; b < NB - 1; ++b) {
+            const bool fin = last && bi == b;
+#pragma unroll
+            for (int m = 0; m < NM; ++m)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) done[b][m][r] = fin ? acc[m][r] : done[b][m][r];
+          }
+#pragma unroll
+          for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[m][r] = last ? 0.0f : acc[m][r];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int bi = 0; bi < NB; ++bi) {
+    f32x4_t tot[NM];
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+      tot[m] = acc[m];
+#pragma unroll
+      for (int b = 0; b < NB - 1; ++b) tot[m] = bi == b ? done[b][m] : tot[m];
+    }
+    const int ch = ch0 + bi * 16;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int t = 4 * q + r;
+      if (t < nt) {
+        const int slot = row0 + t;
+        if constexpr (GATED) {
+          a.out[(int64_t)slot * a.out_ld + ch] =
+              gated_act_bf16(a.act, bf16_round(tot[0][r]), bf16_round(tot[1][r]));
+        } else {
+          const int64_t orow = a.out_by_flat ? rec[4 + t] : slot;
+          a.out[orow * a.out_ld + ch] = f32_to_bf16(tot[0][r]);
+        }
+      }
+    }
+  }
+}
+
 // Tokens per pass follow the expert's row count: 4 (GG = 4) for experts
 // with at most kStreamTT4Rows rows, else 8 (GG = 2).  LDS is sized
 // for 8.
@@ -852,7 +1121,7 @@ __global__ __launch_bounds__(64 * MLXR_STREAM_WAVES) void qgemm_stream_kernel(
     QGemmArgs a, int tiles_n, QGemmArgs a2, int units1, int items1, int rows2) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   Unit u;
-  if (!decode_unit(a, tiles_n, units1, items1, rows2, u)) return;
+  if (!decode_unit<kWorkRows>(a, tiles_n, units1, items1, rows2, u)) return;
   const QGemmArgs& A = u.shared ? a2 : a;
   // The MFMA form follows the expert's row count (not the item's), so every
   // token of an expert is summed in the same order, wherever its item
@@ -864,6 +1133,25 @@ __global__ __launch_bounds__(64 * MLXR_STREAM_WAVES) void qgemm_stream_kernel(
   else
     stream_body<BITS, GATED, 8, D8, NB, KS>(A, u.rec, u.wk, u.fr0, u.fr1, u.tile, smem,
                                             threadIdx.x, blockDim.x, nullptr, 0);
+}
+
+// The same over wide items (16 rows): an item of an expert of more than 8 rows
+// runs in the wide form.
+template <int BITS, bool GATED, int D, int D8, int NB>
+__global__ __launch_bounds__(64 * MLXR_STREAM_WAVES, 3) void qgemm_stream_wide_kernel(
+    QGemmArgs a, int tiles_n, QGemmArgs a2, int units1, int items1, int rows2) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  Unit u;
+  if (!decode_unit<kWorkRowsWide>(a, tiles_n, units1, items1, rows2, u)) return;
+  const QGemmArgs& A = u.shared ? a2 : a;
+  if (u.wk.w <= kStreamTT4Rows)
+    stream_body<BITS, GATED, 4, D, NB, 1>(A, u.rec, u.wk, u.fr0, u.fr1, u.tile, smem,
+                                          threadIdx.x, blockDim.x, nullptr, 0);
+  else if (u.wk.w <= kWorkRows)
+    stream_body<BITS, GATED, 8, D8, NB, 1>(A, u.rec, u.wk, u.fr0, u.fr1, u.tile, smem,
+                                           threadIdx.x, blockDim.x, nullptr, 0);
+  else
+    stream16_body<BITS, GATED, NB>(A, u.rec, u.wk, u.tile, smem);
 }
 
 // q ? b : c, field by field: every field a scalar select, so the chosen
@@ -885,6 +1173,7 @@ __device__ __forceinline__ QGemmArgs pick_args(bool q, const QGemmArgs& b, const
   r.num_active = q ? b.num_active : c.num_active;
   r.work = q ? b.work : c.work;
   r.num_work = q ? b.num_work : c.num_work;
+  r.work_rows = q ? b.work_rows : c.work_rows;
   r.tiles = q ? b.tiles : c.tiles;
   r.num_tiles = q ? b.num_tiles : c.num_tiles;
   r.sorted = q ? b.sorted : c.sorted;
@@ -931,7 +1220,7 @@ __global__ __launch_bounds__(1024) void qgemm_down_combine_kernel(
   // these stores)
   if ((int)threadIdx.x < nsub * 2)
     reinterpret_cast<u32x4_t*>(yl)[threadIdx.x] = u32x4_t{0u, 0u, 0u, 0u};
-  const int32_t* rec = a.work + (int64_t)kWorkInts * (sh ? 0 : sub);
+  const int32_t* rec = a.work + (int64_t)work_ints(kWorkRows) * (sh ? 0 : sub);
   int4 wk = *reinterpret_cast<const int4*>(rec);
   int4 fr0 = *reinterpret_cast<const int4*>(rec + 4);
   int4 fr1 = *reinterpret_cast<const int4*>(rec + 8);
@@ -1039,6 +1328,30 @@ StreamShape stream_shape(const QGemmArgs& a, int64_t all_items) {
   return StreamShape{nb, ks, tiles_n, base_lds + (ks > 1 ? red_lds : 0)};
 }
 
+// ... of the wide items' kernel: no K-slices (the grids are large); LDS for the
+// larger of the 8- and the 16-token form.
+StreamShape stream_wide_shape(const QGemmArgs& a, int64_t all_items) {
+  constexpr int kWaves = MLXR_STREAM_WAVES;
+  const int groups = a.K / 64;
+  const int64_t per_tile = a.N / (16 * kWaves);
+  int nb = 1;
+  if (!a.gated && a.K <= kWideWhole && per_tile % 2 == 0 &&
+      all_items * (per_tile / 2) >= kStreamSlots)
+    nb = 2;
+  const size_t sb_lds = (size_t)kWaves * (a.gated ? 2 : 1) * 2 * nb * 16 * groups * 2;
+  const size_t ks = a.K <= kWideWhole ? a.K : kWideSlice;
+  const size_t lds8 =
+      ((size_t)8 * (a.K + 8) * 2 + 16 + (size_t)groups * 8 * 4 + 15) & ~size_t(15);
+  const size_t lds16 = (size_t)16 * (ks + 8) * 2 + ks / 64 * 16 * 4;
+  return StreamShape{nb, 1, (int)(per_tile / nb),
+                     std::max(lds8, lds16) + ((sb_lds + 15) & ~size_t(15))};
+}
+
+// (defined last: its kernels follow the others in the code object)
+hipError_t launch_stream_wide(const QGemmArgs& a, const QGemmArgs& b, int64_t max_items,
+                              int64_t items2, int64_t shared_rows, const char* profile,
+                              hipStream_t s);
+
 }  // namespace
 
 hipError_t launch_qgemm(const QGemmArgs& a, int64_t total_rows,
@@ -1048,7 +1361,7 @@ hipError_t launch_qgemm(const QGemmArgs& a, int64_t total_rows,
   if (!profile) profile = a.gated ? "qgemm_gated" : "qgemm_down";
   // a folded second problem: the same projection shape and format, its
   // items (or M-tiles) beside the routed ones in the same grid
-  const int64_t items2 = shared ? (shared_rows + kWorkRows - 1) / kWorkRows : 0;
+  const int64_t items2 = shared ? (shared_rows + a.work_rows - 1) / a.work_rows : 0;
   if (shared && (shared->N != a.N || shared->K != a.K ||
                  shared->bits != a.bits || shared->gated != a.gated))
     return hipErrorInvalidValue;
@@ -1071,6 +1384,8 @@ hipError_t launch_qgemm(const QGemmArgs& a, int64_t total_rows,
   const int64_t all_items = max_items + items2;
   // (dense bf16 weights, bits 16, take the split-K kernel below)
   if (stream_eligible(a, b, all_items)) {
+    if (a.work_rows == kWorkRowsWide)
+      return launch_stream_wide(a, b, max_items, items2, shared_rows, profile, s);
     constexpr int kWaves = MLXR_STREAM_WAVES;
     const StreamShape sh = stream_shape(a, all_items);
     const int nb = sh.nb, ks = sh.ks, tiles_n = sh.tiles_n;
@@ -1193,7 +1508,7 @@ hipError_t launch_qgemm_down_combine(const QGemmArgs& a, int64_t K, int64_t max_
   if (a.gated || (a.bits != 4 && a.bits != 8) || K < 1 ||
       (shared && (shared->N != a.N || shared->K != a.K || shared->bits != a.bits ||
                   shared->gated)) ||
-      (c.w_bf16 && !c.bf16) || (shared && !c.shared_logit))
+      (c.w_bf16 && !c.bf16) || (shared && !c.shared_logit) || a.work_rows != kWorkRows)
     return hipSuccess;
   const int64_t items2 = shared ? 1 : 0;
   const int64_t all_items = max_items + items2;
@@ -1251,5 +1566,39 @@ hipError_t launch_qgemm_down_combine(const QGemmArgs& a, int64_t K, int64_t max_
   *done = true;
   return hipGetLastError();
 }
+
+namespace {
+
+hipError_t launch_stream_wide(const QGemmArgs& a, const QGemmArgs& b, int64_t max_items,
+                              int64_t items2, int64_t shared_rows, const char* profile,
+                              hipStream_t s) {
+  constexpr int kWaves = MLXR_STREAM_WAVES;
+  const StreamShape sh = stream_wide_shape(a, max_items + items2);
+  const int items1 = (int)max_items, units1 = (int)(max_items * sh.tiles_n);
+  const dim3 grid((unsigned)(units1 + items2 * sh.tiles_n));
+  ProfileScope prof(profile, s);
+#define MLXR_QW(B, G, D, D8, NB)                                    \
+  qgemm_stream_wide_kernel<B, G, D, D8, NB>                         \
+      <<<grid, 64 * kWaves, sh.lds, s>>>(a, sh.tiles_n, b, units1, items1, (int)shared_rows)
+  if (a.bits == 4) {
+    if (a.gated)
+      MLXR_QW(4, true, MLXR_STREAM_DEPTH4G, MLXR_STREAM_DEPTH4G_TT8, 1);
+    else if (sh.nb == 2)
+      MLXR_QW(4, false, MLXR_STREAM_DEPTH4, MLXR_STREAM_DEPTH4_TT8, 2);
+    else
+      MLXR_QW(4, false, MLXR_STREAM_DEPTH4, MLXR_STREAM_DEPTH4_TT8, 1);
+  } else {
+    if (a.gated)
+      MLXR_QW(8, true, MLXR_STREAM_DEPTH8G, MLXR_STREAM_DEPTH8G_TT8, 1);
+    else if (sh.nb == 2)
+      MLXR_QW(8, false, MLXR_STREAM_DEPTH8, MLXR_STREAM_DEPTH8_TT8, 2);
+    else
+      MLXR_QW(8, false, MLXR_STREAM_DEPTH8, MLXR_STREAM_DEPTH8_TT8, 1);
+  }
+#undef MLXR_QW
+  return hipGetLastError();
+}
+
+}  // namespace
 
 }  // namespace mlxr_moe

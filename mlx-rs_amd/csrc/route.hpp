@@ -246,9 +246,9 @@ __device__ __forceinline__ void block_exclusive_scan(const int (&v)[NV],
 // Work items per expert of cnt rows, listed long form first: the items of
 // experts above kStreamTT4Rows rows (the streaming GEMM's slower 8-token
 // form) take positions [0, total_long), the others follow.
-__device__ __forceinline__ void work_counts(int cnt, bool expert, int& nw_long,
-                                            int& nw_short) {
-  const int nw = expert ? (cnt + kWorkRows - 1) / kWorkRows : 0;
+__device__ __forceinline__ void work_counts(int cnt, bool expert, int work_rows,
+                                            int& nw_long, int& nw_short) {
+  const int nw = expert ? (cnt + work_rows - 1) / work_rows : 0;
   nw_long = cnt > kStreamTT4Rows ? nw : 0;
   nw_short = cnt > kStreamTT4Rows ? 0 : nw;
 }
@@ -259,6 +259,7 @@ __device__ __forceinline__ void work_counts(int cnt, bool expert, int& nw_long,
 // argsort.  Ids of -1 are left out silently; other ids outside [0, E) are
 // left out and flag *status.  Every thread of the 1024-thread workgroup
 // must call it.  Three barriers.
+template <int WR>  // rows per work item (b.work_rows)
 __device__ void block_dispatch(int id_in, int n, int E, int tile_rows,
                                const DispatchBuffers& b, DispatchScratch* ls) {
   constexpr int kWaves = kDispatchBlock / 64;
@@ -298,7 +299,7 @@ __device__ void block_dispatch(int id_in, int n, int E, int tile_rows,
   // M-tiles
   const int has = (tid < E && cnt > 0) ? 1 : 0;
   int nw_long, nw_short;
-  work_counts(cnt, tid < E, nw_long, nw_short);
+  work_counts(cnt, tid < E, WR, nw_long, nw_short);
   const int nw = nw_long + nw_short;
   const int nt = tid < E ? (cnt + tile_rows - 1) / tile_rows : 0;
   int ex[5], tot[5];
@@ -315,8 +316,7 @@ __device__ void block_dispatch(int id_in, int n, int E, int tile_rows,
     const int pos = ls->off[id] + rank;
     b.sorted[pos] = tid;
     b.inv[tid] = pos;
-    b.work[kWorkInts * (ls->wpos[id] + rank / kWorkRows) + 4 +
-           rank % kWorkRows] = tid;
+    b.work[work_ints(WR) * (ls->wpos[id] + rank / WR) + 4 + rank % WR] = tid;
   }
   if (tid < E) {
     b.counts[tid] = cnt;
@@ -324,10 +324,10 @@ __device__ void block_dispatch(int id_in, int n, int E, int tile_rows,
   }
   if (has) b.active[apos] = tid;
   for (int j = 0; j < nw; ++j) {
-    int32_t* w = b.work + kWorkInts * (wpos + j);
+    int32_t* w = b.work + work_ints(WR) * (wpos + j);
     w[0] = tid;
-    w[1] = off + j * kWorkRows;
-    w[2] = min(kWorkRows, cnt - j * kWorkRows);
+    w[1] = off + j * WR;
+    w[2] = min(WR, cnt - j * WR);
     w[3] = cnt;
   }
   for (int j = 0; j < nt; ++j) {
@@ -373,12 +373,14 @@ __device__ void wave_dispatch(int id_in, int n, int E, int tile_rows,
     const uint64_t bal = __ballot(on);
     match &= on ? bal : ~bal;
   }
+  constexpr int wr = kWorkRows, ws = 3;                     // (work_rows_for: n > 64 if wide)
+  static_assert(1 << ws == wr, "a shift");
   const int r = __popcll(match & ((1ull << lane) - 1ull));  // rank among equals
   const int c = ok ? __popcll(match) : 0;                   // the expert's rows
   const bool leader = ok && r == 0;
   // long-form items over all experts: the short-form items start after them
   const uint32_t wl_own =
-      leader && c > kStreamTT4Rows ? (uint32_t)((c + kWorkRows - 1) / kWorkRows) : 0u;
+      leader && c > kStreamTT4Rows ? (uint32_t)((c + wr - 1) >> ws) : 0u;
   const int tot_long = (int)readlane_u32(wave_incl_scan(wl_own), 63);
   for (int e = lane; e < E; e += 64) ls->cnt[e] = 0;
   if (leader) ls->cnt[id] = c;
@@ -388,7 +390,7 @@ __device__ void wave_dispatch(int id_in, int n, int E, int tile_rows,
   for (int e0 = 0; e0 < E; e0 += 64) {
     const int e = e0 + lane;
     const int ce = e < E ? ls->cnt[e] : 0;
-    const int nw = (ce + kWorkRows - 1) / kWorkRows;
+    const int nw = (ce + wr - 1) >> ws;
     const int nt = (ce + tile_rows - 1) / tile_rows;
     const bool lng = ce > kStreamTT4Rows;
     const uint32_t pa = (uint32_t)ce | (ce > 0 ? 1u << 8 : 0u) |
@@ -409,10 +411,10 @@ __device__ void wave_dispatch(int id_in, int n, int E, int tile_rows,
       ls->item[e] = first;
       b.active[(xa >> 8) & 0xffu] = e;
       for (int j = 0; j < nw; ++j) {
-        int32_t* w = b.work + kWorkInts * (first + j);
+        int32_t* w = b.work + work_ints(wr) * (first + j);
         w[0] = e;
-        w[1] = off + j * kWorkRows;
-        w[2] = min(kWorkRows, ce - j * kWorkRows);
+        w[1] = off + j * wr;
+        w[2] = min(wr, ce - j * wr);
         w[3] = ce;
       }
       const int tb = (int)((xa >> 16) & 0xffu);
@@ -426,7 +428,7 @@ __device__ void wave_dispatch(int id_in, int n, int E, int tile_rows,
     const int pos = ls->pos[id] + r;
     b.sorted[pos] = lane;
     b.inv[lane] = pos;
-    b.work[kWorkInts * (ls->item[id] + r / kWorkRows) + 4 + r % kWorkRows] = lane;
+    b.work[work_ints(wr) * (ls->item[id] + (r >> ws)) + 4 + (r & (wr - 1))] = lane;
   }
   if (lane == 0) {
     b.offsets[E] = (int)(carry_a & 0xffu);

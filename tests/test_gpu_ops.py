@@ -400,6 +400,46 @@ def test_gather_qmm_register_tiles(pkg, dev, bits, N, K, offset, counts):
         assert bool(((got[r, 0].double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("E,N,K", [
+    (64, 128, 256), (64, 64, 512), (64, 128, 768), (64, 192, 1536), (64, 128, 2048),
+    (64, 64, 3072), (64, 64, 4096), (64, 128, 1792), (8, 64, 2048), (64, 128, 320)])
+def test_gather_qmm_wide_items(pkg, dev, bits, E, N, K):
+    """Calls of 6 to 16 rows per expert (work items of 16 rows): experts of 1
+    to 40 rows, x staged whole and in slices, input dims and expert counts
+    that keep the 8-row items or the split-K kernel.  Within f32 sums and one
+    bf16 rounding of a 64-bit product with the weights code * scale + bias."""
+    base = [16, 17, 9, 8, 1, 33, 12, 4, 5, 0, 15, 40, 2, 7, 10, 3]
+    counts = (base * (E // 16 + 1))[:E] if E >= 16 else [16, 17, 9, 8, 1, 33, 12, 4]
+    B = sum(counts)
+    assert 6 * E <= B and not pkg.ops.gather_qmm_tiled(B, E)
+    g = torch.Generator(device=dev)
+    g.manual_seed(K + N + bits)
+    ids = torch.repeat_interleave(torch.arange(E, device=dev), torch.tensor(counts, device=dev))
+    ids = ids[torch.randperm(B, generator=g, device=dev)].to(torch.int32)
+    x = torch.randn((B, 1, K), generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn((E, N, K), generator=g, device=dev) * 0.02).to(torch.bfloat16)
+    wq, sc, bi = pkg.ops.quantize(w, 64, bits)
+    got = pkg.ops.gather_qmm(x, wq, sc, bi, None, ids, True, 64, bits)
+    code = (wq.long()[..., None] >> torch.arange(0, 32, bits, device=dev)) & (2 ** bits - 1)
+    wd = (code.reshape(E, N, -1, 64).double() * sc.double()[..., None] +
+          bi.double()[..., None]).reshape(E, N, K)
+    xd = x[:, 0].double()
+    for e in range(E):
+        r = (ids == e).nonzero()[:, 0]
+        want = xd[r] @ wd[e].t()
+        # the offset form sums 16 s x (1 + c / 16) and (b - 16 s) x apart: f32
+        # sums of K products no larger than |x| (31 s + |b|)
+        size = (xd[r].abs().reshape(-1, K // 64, 64).sum(-1) @
+                (31 * sc[e].double().abs() + bi[e].double().abs()).t())
+        if bits == 8:
+            size = xd[r].abs() @ wd[e].abs().t() + 2 * (
+                xd[r].abs().reshape(-1, K // 64, 64).sum(-1) @ (
+                    255 * sc[e].double().abs() + bi[e].double().abs()).t())
+        bound = 2.0 ** -8 * want.abs() + (64 + K // 64) * 2.0 ** -24 * size
+        assert bool(((got[r, 0].double() - want).abs() <= bound).all()), (e, counts[e])
+
+
 def test_gather_qmm_out_of_range_index(pkg, orc, dev):
     wq, sc, bi = _qbank(pkg, orc, 4, 64, 64, 4, dev, 3)
     x = torch.ones((3, 1, 64), dtype=torch.bfloat16, device=dev)

@@ -69,9 +69,12 @@ DispatchBuffers carve_dispatch(Carve& c, int64_t n, int64_t E,
   b.active = c.take<int32_t>(E);
   b.num_active = c.take<int32_t>(1);
   // (room for the items of either size)
-  b.work = c.take<int32_t>(
-      std::max(work_ints(kWorkRows) * dispatch_max_work(n, E, kWorkRows),
-               work_ints(kWorkRowsWide) * dispatch_max_work(n, E, kWorkRowsWide)));
+  const int64_t ints = work_ints(kWorkRows) * dispatch_max_work(n, E, kWorkRows);
+  const int64_t wide = std::max(
+      ints, work_ints(kWorkRowsWide) * dispatch_max_work(n, E, kWorkRowsWide));
+  b.work = c.take<int32_t>(wide);
+  c.wide_room += (((size_t)wide * 4 + 255) & ~size_t(255)) -
+                 (((size_t)ints * 4 + 255) & ~size_t(255));
   b.work_rows = kWorkRows;
   b.num_work = c.take<int32_t>(1);
   b.work_first = c.take<int32_t>(E);

@@ -132,7 +132,7 @@ constexpr int kWorkRowsWide = 16;
 // Work item record: expert, first sorted slot, rows (<= work_rows), rows of
 // the whole expert, then the flat row index (sorted[slot]) of each of the
 // item's slots (unset past rows).  A GEMM workgroup learns its task, and
-// where its x rows live, from these 48 bytes without a dependent load.
+// where its x rows live, from these bytes without a dependent load.
 __host__ __device__ constexpr int work_ints(int work_rows) { return 4 + work_rows; }
 // The streaming decode GEMM runs the items of experts with at most this many
 // rows in its 4-token MFMA form, the others in the 8-token form (longer per

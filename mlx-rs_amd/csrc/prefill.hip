@@ -50,8 +50,7 @@ namespace tile256 {
 // 128 rows of dense bf16 weights: 128 columns, 4 waves of 64 x 64, two stages
 // in 64 KB of LDS, so that two workgroups share a CU and one's barrier waits
 // and staging overlap the other's MFMAs (c8 T=2048 gate/up 237 us with 256
-// columns and 8 waves, 232 so).  Quantised weights run the 64-row tiles of
-// prefill_reg.hip up to the 256-row ones.
+// columns and 8 waves, 232 so).
 namespace tile128n {
 #define MLXR_PF_TILE_ROWS 128
 #define MLXR_PF_MBLOCKS 2

@@ -133,15 +133,10 @@ int run_gather(const char* op, const void* x, int64_t x_batch, int64_t M,
   int32_t* ids = c.take<int32_t>(R);
   int32_t* xrow = c.take<int32_t>(R);
   DispatchBuffers db = carve_dispatch(c, R, E, status);
-  db.work_rows = work_rows_for(R, E, K, 0, bits);
   uint16_t* ob = static_cast<uint16_t*>(out);
   st = from_hip(launch_gather_prep(lhs_indices, rhs_indices, B, M, x_batch, E,
                                    N, ids, xrow, ob, status, s),
                 (o + " prep").c_str());
-  if (st.ok)
-    st = from_hip(launch_dispatch(ids, R, E, prefill_tile_rows(R, E, bits), db, false, s),
-                  (o + " dispatch").c_str());
-  if (!st.ok) return finish(st);
   QGemmArgs a{};
   a.x = static_cast<const uint16_t*>(x);
   a.x_ld = K;
@@ -154,7 +149,6 @@ int run_gather(const char* op, const void* x, int64_t x_batch, int64_t M,
   a.num_active = db.num_active;
   a.work = db.work;
   a.num_work = db.num_work;
-  a.work_rows = db.work_rows;
   a.tiles = db.tiles;
   a.num_tiles = db.num_tiles;
   a.sorted = db.sorted;
@@ -170,6 +164,12 @@ int run_gather(const char* op, const void* x, int64_t x_batch, int64_t M,
   a.out_ld = N;
   a.out_by_flat = true;
   a.gated = false;
+  db.work_rows = work_rows_for(R, E, {&a});
+  a.work_rows = (uint8_t)db.work_rows;
+  if (st.ok)
+    st = from_hip(launch_dispatch(ids, R, E, prefill_tile_rows(R, E, bits), db, false, s),
+                  (o + " dispatch").c_str());
+  if (!st.ok) return finish(st);
   return finish(from_hip(launch_qgemm(a, R, dispatch_max_work(R, E, db.work_rows),
                                       nn::use_prefill_path(R, E, bits), s),
                          op));

@@ -6,6 +6,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <initializer_list>
 #include <string>
 
 namespace mlxr_moe {
@@ -147,23 +148,12 @@ int64_t dispatch_max_tiles(int64_t n, int64_t E, int tile_rows);
 inline int64_t dispatch_max_work(int64_t n, int64_t E, int work_rows = kWorkRows) {
   return (E < n ? E : n) + n / work_rows;
 }
-// Rows per work item of a call whose GEMMs have input dims K0 and K1 (0: one
-// GEMM): wide items from MLXR_WIDE_ITEM_ROWS rows per expert, where more than
-// one in seven experts has over kWorkRows rows: at 6 rows per expert a step of
-// c2 (T = 96) went from 117 us to 114, c6 (T = 200) 193 to 188; with fewer, the
-// 8-row items' kernel covers nearly every expert in one item and has the
-// smaller LDS and register footprint.  For quantised weights and
-// input dims that the wide form stages (stream16_body); more than 64 rows (the
-// one-wave sort of fewer makes 8-row items).
+// The least rows of a call with wide items (work_rows_for).
 #ifndef MLXR_WIDE_ITEM_ROWS
 #define MLXR_WIDE_ITEM_ROWS 6
 #endif
-constexpr int kWideWhole = 1536, kWideSlice = 1024;
-inline int work_rows_for(int64_t n, int64_t E, int64_t K0, int64_t K1, int bits) {
-  const auto fits = [](int64_t k) { return k <= kWideWhole || k % kWideSlice == 0; };
-  return bits != 16 && n > 64 && n >= MLXR_WIDE_ITEM_ROWS * E && fits(K0) && fits(K1)
-             ? kWorkRowsWide
-             : kWorkRows;
+inline bool wide_items_possible(int64_t n, int64_t E) {
+  return n > 64 && n >= MLXR_WIDE_ITEM_ROWS * E;
 }
 // Clears a workspace status word with a one-thread kernel (no memset node,
 // so the call stays valid under stream capture).
@@ -220,7 +210,7 @@ struct QGemmArgs {
   const int32_t* row_map;
   int32_t row_div;
   bool x_by_slot;
-  uint8_t work_rows;       // rows per work item (in what would be padding)
+  uint8_t work_rows;       // rows per work item (the launcher's; in padding)
   const int32_t* offsets;  // [E+1] slot range of each expert
   const int32_t* active;   // [E] experts with rows
   const int32_t* num_active;
@@ -241,6 +231,19 @@ struct QGemmArgs {
   bool out_by_flat;        // out row of slot p = its flat row (else p)
   bool gated;              // out = act(x.w0, x.w1)
 };
+// Rows per work item of a dispatch of n rows over E experts for these GEMMs
+// (shapes, weights and formats filled in; a folded shared expert's among
+// them): wide items from MLXR_WIDE_ITEM_ROWS rows per expert, where more than
+// one in seven experts has over kWorkRows rows: at 6 rows per expert a step of
+// c2 (T = 96) went from 117 us to 114, c6 (T = 200) 193 to 188; with fewer, the
+// 8-row items' kernel covers nearly every expert in one item and has the
+// smaller LDS and register footprint.  Only where every GEMM runs the streaming
+// kernel, without K-slices, with 8-row items: then the sums are those of 8-row
+// items, and the grid is large enough for items twice as long (a one-expert
+// MLP of d 2048, f 512 at T = 200 took 35.4 us in wide items, 33.3 in K-sliced
+// 8-row ones).  Input dims that the wide form stages (stream16_body); more
+// than 64 rows (the one-wave sort of fewer makes 8-row items).
+int work_rows_for(int64_t n, int64_t E, std::initializer_list<const QGemmArgs*> gemms);
 constexpr int32_t kActSwiglu = 0;  // silu(g) * u  (Qwen3.5/3.6 experts)
 constexpr int32_t kActGeglu = 1;   // gelu_approx(g) * u  (gemma4 experts)
 // Largest input dim (K) of a projection: 8 waves x 8 groups of 64.

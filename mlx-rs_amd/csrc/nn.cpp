@@ -68,11 +68,10 @@ DispatchBuffers carve_dispatch(Carve& c, int64_t n, int64_t E,
   b.inv = c.take<int32_t>(n);
   b.active = c.take<int32_t>(E);
   b.num_active = c.take<int32_t>(1);
-  // (room for the items of either size, where wide ones can be chosen: input
-  // dims of 64 fit them, and bits only rule them out)
+  // (room for the items of either size, where wide ones can be chosen)
   const int64_t ints = work_ints(kWorkRows) * dispatch_max_work(n, E, kWorkRows);
   const int64_t wide =
-      work_rows_for(n, E, 64, 64, 4) == kWorkRows
+      !wide_items_possible(n, E)
           ? ints
           : std::max(ints, work_ints(kWorkRowsWide) * dispatch_max_work(n, E, kWorkRowsWide));
   b.work = c.take<int32_t>(wide);
@@ -121,6 +120,19 @@ QWeights qw(const mlxr_moe_qlinear& q) {
                   static_cast<const uint16_t*>(q.biases)};
 }
 
+// A GEMM as work_rows_for looks at it.
+QGemmArgs gemm_shape(const QWeights& w0, const QWeights& w1, bool gated, int64_t N,
+                     int64_t K, int bits) {
+  QGemmArgs g{};
+  g.w0 = w0;
+  g.w1 = w1;
+  g.gated = gated;
+  g.N = (int32_t)N;
+  g.K = (int32_t)K;
+  g.bits = bits;
+  return g;
+}
+
 }  // namespace
 
 // ------------------------------------------------------------- SwigluMlp
@@ -146,7 +158,9 @@ Status SwigluMlp::forward(const uint16_t* x, int64_t T, uint16_t* y,
                           Carve& ws, int32_t* status, hipStream_t s) const {
   const int64_t d = gate_.input_dims, f = gate_.output_dims;
   DispatchBuffers db = carve_dispatch(ws, T, 1, status);
-  db.work_rows = work_rows_for(T, 1, d, f, gate_.bits);
+  const QGemmArgs gs = gemm_shape(qw(gate_), qw(up_), true, f, d, gate_.bits);
+  const QGemmArgs ds = gemm_shape(qw(down_), QWeights{}, false, d, f, gate_.bits);
+  db.work_rows = work_rows_for(T, 1, {&gs, &ds});
   uint16_t* act = ws.take<uint16_t>(T * f);
   Status st = from_hip(launch_dispatch_identity(T, prefill_tile_rows(T, 1, gate_.bits), db, s),
                        "shared_expert dispatch");
@@ -299,13 +313,22 @@ Status SwitchFfn::forward(const uint16_t* x, int64_t T, const int32_t* indices,
   const int64_t E = sw_.E;
   const int64_t n = T * K;
   DispatchBuffers db = carve_dispatch(ws, n, E, status);
-  db.work_rows = work_rows_for(n, E, sw_.d, sw_.f, sw_.bits);
+  db.work_rows = work_rows(n, nullptr);
   // (the dispatch clears *status first: no launch of its own for that)
   Status st = from_hip(
       launch_dispatch(indices, n, E, prefill_tile_rows(n, E, sw_.bits), db, true, s),
       "switch_mlp dispatch");
   if (!st.ok) return st;
   return experts(x, T, K, db, y, ws, s, nullptr, dc, combined);
+}
+
+int SwitchFfn::work_rows(int64_t n, const SharedFold* fold) const {
+  const QGemmArgs g = gemm_shape(sw_.gate, sw_.up, true, sw_.f, sw_.d, sw_.bits);
+  const QGemmArgs h = gemm_shape(sw_.down, QWeights{}, false, sw_.d, sw_.f, sw_.bits);
+  if (!fold) return work_rows_for(n, sw_.E, {&g, &h});
+  const QGemmArgs g2 = gemm_shape(fold->gate, fold->up, true, sw_.f, sw_.d, sw_.bits);
+  const QGemmArgs h2 = gemm_shape(fold->down, QWeights{}, false, sw_.d, sw_.f, sw_.bits);
+  return work_rows_for(n, sw_.E, {&g, &h, &g2, &h2});
 }
 
 // The expert products given the dispatch: gate and up gather_qmm fused with
@@ -523,8 +546,14 @@ Status Qwen35MoeBlock::forward(const uint16_t* x, int64_t T, void* out,
   if (shared) SwigluMlp::plan(ws, T, d, b_.shared_expert_intermediate_size);
   uint16_t* y = ws.take<uint16_t>(T * K * d);
   DispatchBuffers db = carve_dispatch(ws, T * K, E, status);
-  db.work_rows =
-      work_rows_for(T * K, E, d, b_.moe_intermediate_size, b_.switch_mlp.gate_proj.bits);
+  const SplitSwitchFfn mlp(b_.switch_mlp);
+  const SwigluMlp smlp(b_.shared_gate_proj, b_.shared_up_proj,
+                       b_.shared_down_proj);
+  // on the decode kernels the shared expert rides in the routed launches
+  const bool fold = shared && mlp.can_fold(smlp, T, K);
+  SharedFold sf{};
+  if (fold) sf = smlp.fold(shared_ws, T, sy);
+  db.work_rows = mlp.work_rows(T * K, fold ? &sf : nullptr);
   // gate.forward + shared_expert_gate.forward (moe.rs:118,123) in one pass.
   RouterWeights rw = router_weights_f32(
       b_.gate_weight, shared ? b_.shared_expert_gate_weight : nullptr);
@@ -552,17 +581,10 @@ Status Qwen35MoeBlock::forward(const uint16_t* x, int64_t T, void* out,
                              db, s, route_counter),
                 "router top-k / dispatch");
   if (!st.ok) return st;
-  const SplitSwitchFfn mlp(b_.switch_mlp);
-  const SwigluMlp smlp(b_.shared_gate_proj, b_.shared_up_proj,
-                       b_.shared_down_proj);
-  // on the decode kernels the shared expert rides in the routed launches
-  const bool fold = shared && mlp.can_fold(smlp, T, K);
   if (shared && !fold) {
     st = smlp.forward(x, T, sy, shared_ws, status, s);
     if (!st.ok) return st;
   }
-  SharedFold sf{};
-  if (fold) sf = smlp.fold(shared_ws, T, sy);
   // one token: the combine rides in the down launch where it can
   // (top-K picks K different experts: one row per work item)
   const DownCombine dc{wts, false, sy, shared ? logits + E : nullptr, residual, out, bf16,

@@ -146,6 +146,9 @@ class SwitchFfn {
                               hipStream_t s) const;
   static void plan(Carve& ws, int64_t T, int64_t K, int64_t d, int64_t f,
                    int64_t E);
+  // Rows per work item of a dispatch of n rows for the experts' GEMMs, with
+  // `fold` the shared expert's beside them.
+  int work_rows(int64_t n, const SharedFold* fold) const;
   const SwitchWeights& weights() const { return sw_; }
 
  protected:

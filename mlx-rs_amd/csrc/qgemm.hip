@@ -85,6 +85,9 @@ namespace {
 #endif
 
 constexpr int64_t kStreamMinBlocks = MLXR_STREAM_MIN_BLOCKS;
+// The wide items' x stages: whole up to kWideWhole inputs, else kWideSlice at
+// a time.
+constexpr int kWideWhole = 1536, kWideSlice = 1024;
 // 16-channel blocks per wave of the down kernel, at most (1, 2 or 4; the
 // launcher halves it until the grid keeps every slot busy)
 #ifndef MLXR_STREAM_MAX_NB
@@ -292,11 +295,10 @@ __device__ __forceinline__ void decode_body(const QGemmArgs& a, int tile,
     int64_t xrow = 0;
     if (tv) {
       const int slot = row0 + tok;
-      // this lane's flat row from the record (its first eight fetched with the
-      // header)
+      // this lane's flat row from the record (tok < kWorkRows = 8)
       const int f4 = (tok & 3) == 0 ? fr0.x : (tok & 3) == 1 ? fr0.y : (tok & 3) == 2 ? fr0.z : fr0.w;
       const int f8 = (tok & 3) == 0 ? fr1.x : (tok & 3) == 1 ? fr1.y : (tok & 3) == 2 ? fr1.z : fr1.w;
-      const int flat = tok < 4 ? f4 : tok < 8 ? f8 : a.x_by_slot ? 0 : rec[4 + tok];
+      const int flat = tok < 4 ? f4 : f8;
       xrow = a.x_by_slot ? slot : (a.row_map ? a.row_map[flat] : flat / a.row_div);
     }
     f32x4_t acc[CB][NM];
@@ -456,7 +458,7 @@ struct Unit {
   int tile;
   bool shared;
 };
-template <int WR = 0>  // rows per item, or 0: a.work_rows
+template <int WR = kWorkRows>  // rows per item
 __device__ __forceinline__ bool decode_unit(const QGemmArgs& a, int tiles_n,
                                             int units1, int items1, int rows2,
                                             Unit& u) {
@@ -466,15 +468,14 @@ __device__ __forceinline__ bool decode_unit(const QGemmArgs& a, int tiles_n,
   u.tile = v - ai * tiles_n;
   // (the routed record is read unconditionally, item 0's for a shared
   // unit)
-  const int wr = WR ? WR : a.work_rows;
-  u.rec = a.work + (int64_t)work_ints(wr) * (u.shared ? 0 : min(ai, items1 - 1));
+  u.rec = a.work + (int64_t)work_ints(WR) * (u.shared ? 0 : min(ai, items1 - 1));
   u.wk = *reinterpret_cast<const int4*>(u.rec);
   u.fr0 = *reinterpret_cast<const int4*>(u.rec + 4);
   u.fr1 = *reinterpret_cast<const int4*>(u.rec + 8);
   const int n_act = *a.num_work;
   if (u.shared) {
-    const int r0 = wr * ai;
-    u.wk = make_int4(0, r0, min(wr, rows2 - r0), rows2);
+    const int r0 = WR * ai;
+    u.wk = make_int4(0, r0, min(WR, rows2 - r0), rows2);
     u.fr0 = make_int4(r0, r0 + 1, r0 + 2, r0 + 3);
     u.fr1 = make_int4(r0 + 4, r0 + 5, r0 + 6, r0 + 7);
     return true;
@@ -856,7 +857,11 @@ __device__ __forceinline__ void stream_body(const QGemmArgs& a,
 // lane, of group A on lanes 0-31 and B on 32-63, into a word of A and one of B
 // on every lane.  Lane quarter q then supplies codes 16 i + 32 (q & 1) +
 // 8 (q >> 1) .. + 7 of the group to MFMA i of two, and receives tokens
-// 4 q .. 4 q + 3 of channel l % 16: no sums cross lanes.  x is staged whole up
+// 4 q .. 4 q + 3 of channel l % 16: no sums cross lanes.  The sums are those
+// of the 8-token form, bit for bit: an MFMA adds its lane quarters' products
+// quarter by quarter, so MFMA i here is MFMAs 2 i and 2 i + 1 there, and the
+// groups A and the groups B are summed apart (acc[0], acc[1]) and joined at a
+// block's end, as its two halves of the wave are.  x is staged whole up
 // to kWideWhole inputs, else kWideSlice at a time (so that three workgroups
 // still share a CU), NB = 1 then.
 // 12 rows an expert of c7 (T = 190): gate/up 83 us in 8-row items, 72 in these,
@@ -995,10 +1000,10 @@ __device__ __forceinline__ void stream16_body(const QGemmArgs& a, const int32_t*
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
   constexpr int ND = NB > 1 ? NB - 1 : 1;
-  f32x4_t acc[NM], done[ND][NM];
+  f32x4_t acc[2][NM], done[ND][NM];
 #pragma unroll
   for (int m = 0; m < NM; ++m) {
-    acc[m] = zero;
+    acc[0][m] = acc[1][m] = zero;
 #pragma unroll
     for (int b = 0; b < ND; ++b) done[b][m] = zero;
   }
@@ -1065,7 +1070,8 @@ __device__ __forceinline__ void stream16_body(const QGemmArgs& a, const int32_t*
             group_terms<BITS>(sbl[(m * 2) * sbn + si], sbl[(m * 2 + 1) * sbn + si], sc, cb);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-              acc[m][r] = __builtin_fmaf(sc, P[r], __builtin_fmaf(cb, X[r], acc[m][r]));
+              acc[g2][m][r] =
+                  __builtin_fmaf(sc, P[r], __builtin_fmaf(cb, X[r], acc[g2][m][r]));
           }
         }
         if constexpr (NB > 1) {
@@ -1076,12 +1082,16 @@ __device__ __forceinline__ void stream16_body(const QGemmArgs& a, const int32_t*
 #pragma unroll
             for (int m = 0; m < NM; ++m)
 #pragma unroll
-              for (int r = 0; r < 4; ++r) done[b][m][r] = fin ? acc[m][r] : done[b][m][r];
+              for (int r = 0; r < 4; ++r)
+                done[b][m][r] = fin ? acc[0][m][r] + acc[1][m][r] : done[b][m][r];
           }
 #pragma unroll
           for (int m = 0; m < NM; ++m)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[m][r] = last ? 0.0f : acc[m][r];
+            for (int r = 0; r < 4; ++r) {
+              acc[0][m][r] = last ? 0.0f : acc[0][m][r];
+              acc[1][m][r] = last ? 0.0f : acc[1][m][r];
+            }
         }
       }
     }
@@ -1091,7 +1101,7 @@ __device__ __forceinline__ void stream16_body(const QGemmArgs& a, const int32_t*
     f32x4_t tot[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-      tot[m] = acc[m];
+      tot[m] = acc[0][m] + acc[1][m];
 #pragma unroll
       for (int b = 0; b < NB - 1; ++b) tot[m] = bi == b ? done[b][m] : tot[m];
     }
@@ -1121,7 +1131,7 @@ __global__ __launch_bounds__(64 * MLXR_STREAM_WAVES) void qgemm_stream_kernel(
     QGemmArgs a, int tiles_n, QGemmArgs a2, int units1, int items1, int rows2) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   Unit u;
-  if (!decode_unit<kWorkRows>(a, tiles_n, units1, items1, rows2, u)) return;
+  if (!decode_unit(a, tiles_n, units1, items1, rows2, u)) return;
   const QGemmArgs& A = u.shared ? a2 : a;
   // The MFMA form follows the expert's row count (not the item's), so every
   // token of an expert is summed in the same order, wherever its item
@@ -1173,7 +1183,6 @@ __device__ __forceinline__ QGemmArgs pick_args(bool q, const QGemmArgs& b, const
   r.num_active = q ? b.num_active : c.num_active;
   r.work = q ? b.work : c.work;
   r.num_work = q ? b.num_work : c.num_work;
-  r.work_rows = q ? b.work_rows : c.work_rows;
   r.tiles = q ? b.tiles : c.tiles;
   r.num_tiles = q ? b.num_tiles : c.num_tiles;
   r.sorted = q ? b.sorted : c.sorted;
@@ -1328,7 +1337,7 @@ StreamShape stream_shape(const QGemmArgs& a, int64_t all_items) {
   return StreamShape{nb, ks, tiles_n, base_lds + (ks > 1 ? red_lds : 0)};
 }
 
-// ... of the wide items' kernel: no K-slices (the grids are large); LDS for the
+// ... of the wide items' kernel: no K-slices (work_rows_for); LDS for the
 // larger of the 8- and the 16-token form.
 StreamShape stream_wide_shape(const QGemmArgs& a, int64_t all_items) {
   constexpr int kWaves = MLXR_STREAM_WAVES;
@@ -1353,6 +1362,16 @@ hipError_t launch_stream_wide(const QGemmArgs& a, const QGemmArgs& b, int64_t ma
                               hipStream_t s);
 
 }  // namespace
+
+int work_rows_for(int64_t n, int64_t E, std::initializer_list<const QGemmArgs*> gemms) {
+  if (!wide_items_possible(n, E)) return kWorkRows;
+  for (const QGemmArgs* g : gemms)
+    if (!(g->K <= kWideWhole || g->K % kWideSlice == 0) ||
+        !stream_eligible(*g, *g, dispatch_max_work(n, E, kWorkRowsWide)) ||
+        stream_shape(*g, dispatch_max_work(n, E, kWorkRows)).ks > 1)
+      return kWorkRows;
+  return kWorkRowsWide;
+}
 
 hipError_t launch_qgemm(const QGemmArgs& a, int64_t total_rows,
                         int64_t max_items, bool prefill, hipStream_t s,
@@ -1383,9 +1402,9 @@ hipError_t launch_qgemm(const QGemmArgs& a, int64_t total_rows,
   // spreads each block over up to 16 waves.
   const int64_t all_items = max_items + items2;
   // (dense bf16 weights, bits 16, take the split-K kernel below)
+  if (a.work_rows == kWorkRowsWide)
+    return launch_stream_wide(a, b, max_items, items2, shared_rows, profile, s);
   if (stream_eligible(a, b, all_items)) {
-    if (a.work_rows == kWorkRowsWide)
-      return launch_stream_wide(a, b, max_items, items2, shared_rows, profile, s);
     constexpr int kWaves = MLXR_STREAM_WAVES;
     const StreamShape sh = stream_shape(a, all_items);
     const int nb = sh.nb, ks = sh.ks, tiles_n = sh.tiles_n;

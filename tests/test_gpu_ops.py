@@ -440,6 +440,45 @@ def test_gather_qmm_wide_items(pkg, dev, bits, E, N, K):
         assert bool(((got[r, 0].double() - want).abs() <= bound).all()), (e, counts[e])
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("d", [256, 768, 1536, 2048, 4096])
+def test_wide_items_sum_as_eight_row_items(pkg, dev, bits, d):
+    """A row's result does not depend on the item it runs in: experts of 9 to 33
+    rows in one call (16-row items, x staged whole and in slices), and the same
+    rows eight an expert at a time (the 8-token form).  Equal bits, for one
+    projection as an op and for the gated FFN."""
+    E, f = 64, 256
+    counts = [16, 17, 9, 12, 33, 9, 10, 9] * (E // 8)
+    B = sum(counts)
+    assert not pkg.ops.gather_qmm_tiled(B, E)
+    g = torch.Generator(device=dev)
+    g.manual_seed(d + bits)
+
+    def bank(n, k):
+        w = (torch.randn((E, n, k), generator=g, device=dev) * 0.02).to(torch.bfloat16)
+        return pkg.ops.quantize(w, 64, bits)
+
+    ids = torch.repeat_interleave(torch.arange(E, device=dev), torch.tensor(counts, device=dev))
+    x = torch.randn((B, d), generator=g, device=dev).to(torch.bfloat16)
+    first = [sum(counts[:e]) for e in range(E)]
+    gate, up, down = bank(f, d), bank(f, d), bank(d, f)
+    ffn = pkg.nn.SplitSwitchFfn(*[pkg.nn.QuantizedSwitchLinear(*w, 64, bits)
+                                  for w in (gate, up, down)])
+
+    def both(rows):
+        i = ids[rows].to(torch.int32)
+        return (pkg.ops.gather_qmm(x[rows][:, None], *gate, None, i, True, 64, bits)[:, 0],
+                ffn.forward(x[rows], i[:, None])[:, 0])
+
+    perm = torch.randperm(B, generator=g, device=dev)
+    whole = [torch.empty_like(v).index_copy_(0, perm, v) for v in both(perm)]
+    for j in range(5):
+        rows = torch.tensor([first[e] + min(8 * j, counts[e] - 8) + t
+                             for e in range(E) for t in range(8)], device=dev)
+        for w, v in zip(whole, both(rows)):
+            assert torch.equal(w[rows], v), j
+
+
 def test_gather_qmm_out_of_range_index(pkg, orc, dev):
     wq, sc, bi = _qbank(pkg, orc, 4, 64, 64, 4, dev, 3)
     x = torch.ones((3, 1, 64), dtype=torch.bfloat16, device=dev)

@@ -28,6 +28,7 @@ SOURCES = [
     "router.hip",
     "dispatch.hip",
     "qgemm.hip",
+    "qgemm_wide.hip",
     "prefill.hip",
     "prefill_reg.hip",
     "prefill_tall.hip",

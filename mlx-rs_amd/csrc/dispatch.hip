@@ -175,7 +175,7 @@ __device__ __forceinline__ void dispatch_scan_body(int n, int E, int nb, int til
     const int* start = i < tot[2] ? s_wlong : s_wshort;
     const int e = upper_slot(start, E, i), j = i - start[e];
     const int cnt_e = (e + 1 < E ? s_off[e + 1] : total) - s_off[e];
-    int32_t* w = b.work + work_ints(b.work_rows) * i;
+    int32_t* w = b.work + kWorkInts * i;
     w[0] = e;
     w[1] = s_off[e] + j * b.work_rows;
     w[2] = min(b.work_rows, cnt_e - j * b.work_rows);
@@ -232,9 +232,9 @@ __global__ __launch_bounds__(kDispatchBlock) void dispatch_scatter_kernel(
   const int pos = base + r;
   b.sorted[pos] = (int32_t)i;
   b.inv[i] = pos;
-  const int wr = b.work_rows;  // a power of two
-  b.work[work_ints(wr) * (b.work_first[e] + r / wr) + 4 + (r & (wr - 1))] =
-      (int32_t)i;
+  const int t = r & (b.work_rows - 1);  // its place in the item
+  if (t < kWorkRows)
+    b.work[kWorkInts * (b.work_first[e] + (r >> work_shift(b.work_rows))) + 4 + t] = (int32_t)i;
 }
 
 // n <= 1024 ids: the whole sort in one workgroup.
@@ -381,12 +381,12 @@ __global__ __launch_bounds__(256) void dispatch_identity_kernel(
     b.inv[i] = i;
   }
   for (int j = tid; j * b.work_rows < n; j += 256) {
-    int32_t* w = b.work + work_ints(b.work_rows) * j;
+    int32_t* w = b.work + kWorkInts * j;
     w[0] = 0;
     w[1] = j * b.work_rows;
     w[2] = min(b.work_rows, n - j * b.work_rows);
     w[3] = n;
-    for (int i = 0; i < b.work_rows; ++i) w[4 + i] = j * b.work_rows + i;
+    for (int i = 0; i < kWorkRows; ++i) w[4 + i] = j * b.work_rows + i;
   }
 }
 

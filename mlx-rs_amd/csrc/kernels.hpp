@@ -130,11 +130,18 @@ constexpr int kWorkRows = 8;
 // ... and of the wide items (work_rows_for), where experts of more rows are
 // common: the weights are then read once per 16 rows.
 constexpr int kWorkRowsWide = 16;
+// log2 of either
+__host__ __device__ constexpr int work_shift(int work_rows) {
+  return work_rows == kWorkRowsWide ? 4 : 3;
+}
 // Work item record: expert, first sorted slot, rows (<= work_rows), rows of
 // the whole expert, then the flat row index (sorted[slot]) of each of the
-// item's slots (unset past rows).  A GEMM workgroup learns its task, and
-// where its x rows live, from these bytes without a dependent load.
-__host__ __device__ constexpr int work_ints(int work_rows) { return 4 + work_rows; }
+// item's first kWorkRows slots (unset past rows).  A GEMM workgroup learns its
+// task, and where its x rows live, from these 48 bytes without a dependent
+// load; a wide item's kernel looks its rows up in sorted.  (The same record for
+// both, and no more items of 16 rows than of 8: the room does not depend on the
+// choice.)
+constexpr int kWorkInts = 4 + kWorkRows;
 // The streaming decode GEMM runs the items of experts with at most this many
 // rows in its 4-token MFMA form, the others in the 8-token form (longer per
 // item: the dispatch lists their items first, so the long workgroups start
@@ -147,13 +154,6 @@ int64_t dispatch_max_tiles(int64_t n, int64_t E, int tile_rows);
 // Bound on the work items of n flat rows over E experts.
 inline int64_t dispatch_max_work(int64_t n, int64_t E, int work_rows = kWorkRows) {
   return (E < n ? E : n) + n / work_rows;
-}
-// The least rows of a call with wide items (work_rows_for).
-#ifndef MLXR_WIDE_ITEM_ROWS
-#define MLXR_WIDE_ITEM_ROWS 6
-#endif
-inline bool wide_items_possible(int64_t n, int64_t E) {
-  return n > 64 && n >= MLXR_WIDE_ITEM_ROWS * E;
 }
 // Clears a workspace status word with a one-thread kernel (no memset node,
 // so the call stays valid under stream capture).
@@ -214,11 +214,11 @@ struct QGemmArgs {
   const int32_t* offsets;  // [E+1] slot range of each expert
   const int32_t* active;   // [E] experts with rows
   const int32_t* num_active;
-  const int32_t* work;     // work item records (work_ints(work_rows) each)
+  const int32_t* work;     // work item records (kWorkInts each)
   const int32_t* num_work;
   const int32_t* tiles;    // M-tile list (prefill path)
   const int32_t* num_tiles;
-  const int32_t* sorted;   // flat row of each sorted slot (prefill path)
+  const int32_t* sorted;   // flat row of each sorted slot (prefill path, wide items)
   QWeights w0;             // gate (or the only projection)
   QWeights w1;             // up (gated mode only)
   int32_t E, N, K, bits;
@@ -243,6 +243,9 @@ struct QGemmArgs {
 // MLP of d 2048, f 512 at T = 200 took 35.4 us in wide items, 33.3 in K-sliced
 // 8-row ones).  Input dims that the wide form stages (stream16_body); more
 // than 64 rows (the one-wave sort of fewer makes 8-row items).
+#ifndef MLXR_WIDE_ITEM_ROWS
+#define MLXR_WIDE_ITEM_ROWS 6
+#endif
 int work_rows_for(int64_t n, int64_t E, std::initializer_list<const QGemmArgs*> gemms);
 constexpr int32_t kActSwiglu = 0;  // silu(g) * u  (Qwen3.5/3.6 experts)
 constexpr int32_t kActGeglu = 1;   // gelu_approx(g) * u  (gemma4 experts)

@@ -68,15 +68,7 @@ DispatchBuffers carve_dispatch(Carve& c, int64_t n, int64_t E,
   b.inv = c.take<int32_t>(n);
   b.active = c.take<int32_t>(E);
   b.num_active = c.take<int32_t>(1);
-  // (room for the items of either size, where wide ones can be chosen)
-  const int64_t ints = work_ints(kWorkRows) * dispatch_max_work(n, E, kWorkRows);
-  const int64_t wide =
-      !wide_items_possible(n, E)
-          ? ints
-          : std::max(ints, work_ints(kWorkRowsWide) * dispatch_max_work(n, E, kWorkRowsWide));
-  b.work = c.take<int32_t>(wide);
-  c.wide_room += (((size_t)wide * 4 + 255) & ~size_t(255)) -
-                 (((size_t)ints * 4 + 255) & ~size_t(255));
+  b.work = c.take<int32_t>(kWorkInts * dispatch_max_work(n, E));
   b.work_rows = kWorkRows;
   b.num_work = c.take<int32_t>(1);
   b.work_first = c.take<int32_t>(E);

@@ -24,8 +24,6 @@ namespace mlxr_moe {
 struct Carve {
   char* base;
   size_t off = 0;
-  // of off: what the wide work items' records take beyond the 8-row items'
-  size_t wide_room = 0;
   explicit Carve(void* b) : base(static_cast<char*>(b)) {}
   template <class T>
   T* take(int64_t count) {

@@ -24,11 +24,7 @@
 namespace mlxr_moe {
 namespace {
 
-// The caller's bytes and the room of the wide work items' records: up to 8
-// ints an expert (1024 at most) and a little for the shared expert, counted
-// apart so that the T a call may have does not depend on the records' form.
-constexpr size_t kWideRoom = 64 * 1024;
-static __device__ __align__(256) char scratch[MLXR_MOE_NOALLOC_SCRATCH_BYTES + kWideRoom];
+static __device__ __align__(256) char scratch[MLXR_MOE_NOALLOC_SCRATCH_BYTES];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
@@ -88,11 +84,8 @@ extern "C" int mlxr_moe_block_forward_noalloc(const mlxr_moe_block* block,
   const Status st = nn::Qwen35MoeBlock(*block).validate();
   if (!st.ok) return capi_fail(st.what);
   if (T < 0) return capi_fail("block_forward_noalloc: bad T");
-  Carve plan(nullptr);
-  plan.take<int32_t>(1);
-  nn::Qwen35MoeBlock::plan(plan, *block, T);
-  const size_t need = plan.off - plan.wide_room;
-  if (need > (size_t)MLXR_MOE_NOALLOC_SCRATCH_BYTES || plan.wide_room > kWideRoom)
+  const size_t need = mlxr_moe_block_workspace_size(block, T);
+  if (need > (size_t)MLXR_MOE_NOALLOC_SCRATCH_BYTES)
     return capi_fail("block_forward_noalloc: T = " + std::to_string(T) +
                      " needs " + std::to_string(need) +
                      " bytes of scratch, more than the library's " +
@@ -110,5 +103,5 @@ extern "C" int mlxr_moe_block_forward_noalloc(const mlxr_moe_block* block,
   void* ws = scratch_on(dev, &err);
   if (!ws) return capi_fail(err);
   return mlxr_moe_block_forward(block, x, T, out, topk_idx, topk_w, ws,
-                                sizeof(scratch), stream);
+                                MLXR_MOE_NOALLOC_SCRATCH_BYTES, stream);
 }

@@ -421,7 +421,7 @@ __global__ __launch_bounds__(1024) void qgemm_down_combine_kernel(
   // these stores)
   if ((int)threadIdx.x < nsub * 2)
     reinterpret_cast<u32x4_t*>(yl)[threadIdx.x] = u32x4_t{0u, 0u, 0u, 0u};
-  const int32_t* rec = a.work + (int64_t)work_ints(kWorkRows) * (sh ? 0 : sub);
+  const int32_t* rec = a.work + (int64_t)kWorkInts * (sh ? 0 : sub);
   int4 wk = *reinterpret_cast<const int4*>(rec);
   int4 fr0 = *reinterpret_cast<const int4*>(rec + 4);
   int4 fr1 = *reinterpret_cast<const int4*>(rec + 8);
@@ -526,7 +526,7 @@ StreamShape stream_shape(const QGemmArgs& a, int64_t all_items) {
 }  // namespace
 
 int work_rows_for(int64_t n, int64_t E, std::initializer_list<const QGemmArgs*> gemms) {
-  if (!wide_items_possible(n, E)) return kWorkRows;
+  if (n <= 64 || n < MLXR_WIDE_ITEM_ROWS * E) return kWorkRows;
   for (const QGemmArgs* g : gemms)
     if (!(g->K <= kWideWhole || g->K % kWideSlice == 0) ||
         !stream_eligible(*g, *g, dispatch_max_work(n, E, kWorkRowsWide)) ||

@@ -150,7 +150,7 @@ __device__ __forceinline__ bool decode_unit(const QGemmArgs& a, int tiles_n,
   u.tile = v - ai * tiles_n;
   // (the routed record is read unconditionally, item 0's for a shared
   // unit)
-  u.rec = a.work + (int64_t)work_ints(WR) * (u.shared ? 0 : min(ai, items1 - 1));
+  u.rec = a.work + (int64_t)kWorkInts * (u.shared ? 0 : min(ai, items1 - 1));
   u.wk = *reinterpret_cast<const int4*>(u.rec);
   u.fr0 = *reinterpret_cast<const int4*>(u.rec + 4);
   u.fr1 = *reinterpret_cast<const int4*>(u.rec + 8);

@@ -32,8 +32,8 @@ namespace {
 // down 59 and 44.  Steps of c2 at 8, 10 and 14 rows an expert (T = 128, 160,
 // 224): 128, 151, 186 us and 117, 130, 154; c5 at 6 (T = 200) 893 and 810.
 template <int BITS, bool GATED, int NB>
-__device__ __forceinline__ void stream16_body(const QGemmArgs& a, const int32_t* rec, int4 wk,
-                                              int tile, char* smem) {
+__device__ __forceinline__ void stream16_body(const QGemmArgs& a, int4 wk, int tile,
+                                              char* smem) {
   constexpr int TT = 16, D = 3, R = D + 1;
   constexpr int NM = GATED ? 2 : 1, NA = 2 * NM;
   constexpr int NL = BITS / 4;     // 16-byte loads per lane and super-step
@@ -79,13 +79,14 @@ __device__ __forceinline__ void stream16_body(const QGemmArgs& a, const int32_t*
   const int k8 = tid & 127, rh = 8 * (tid >> 7), rows_h = nt - rh;
   int64_t xr[8];
   {
-    const int4 f0 = *reinterpret_cast<const int4*>(rec + 4 + rh);
-    const int4 f1 = *reinterpret_cast<const int4*>(rec + 8 + rh);
-    const int fl[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
-    int32_t rm[8];
+    int32_t fl[8], rm[8];
+    if (!a.x_by_slot) {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) fl[t] = a.sorted[row0 + min(rh + t, nt - 1)];
+    }
     if (!a.x_by_slot && a.row_map) {
 #pragma unroll
-      for (int t = 0; t < 8; ++t) rm[t] = a.row_map[t < rows_h ? fl[t] : rec[4]];
+      for (int t = 0; t < 8; ++t) rm[t] = a.row_map[fl[t]];
     }
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
@@ -279,7 +280,7 @@ __device__ __forceinline__ void stream16_body(const QGemmArgs& a, const int32_t*
           a.out[(int64_t)slot * a.out_ld + ch] =
               gated_act_bf16(a.act, bf16_round(tot[0][r]), bf16_round(tot[1][r]));
         } else {
-          const int64_t orow = a.out_by_flat ? rec[4 + t] : slot;
+          const int64_t orow = a.out_by_flat ? a.sorted[slot] : slot;
           a.out[orow * a.out_ld + ch] = f32_to_bf16(tot[0][r]);
         }
       }
@@ -303,7 +304,7 @@ __global__ __launch_bounds__(64 * MLXR_STREAM_WAVES, 3) void qgemm_stream_wide_k
     stream_body<BITS, GATED, 8, D8, NB, 1>(A, u.rec, u.wk, u.fr0, u.fr1, u.tile, smem,
                                            threadIdx.x, blockDim.x, nullptr, 0);
   else
-    stream16_body<BITS, GATED, NB>(A, u.rec, u.wk, u.tile, smem);
+    stream16_body<BITS, GATED, NB>(A, u.wk, u.tile, smem);
 }
 
 // ... of the wide items' kernel: no K-slices (work_rows_for); LDS for the

@@ -248,7 +248,7 @@ __device__ __forceinline__ void block_exclusive_scan(const int (&v)[NV],
 // form) take positions [0, total_long), the others follow.
 __device__ __forceinline__ void work_counts(int cnt, bool expert, int work_rows,
                                             int& nw_long, int& nw_short) {
-  const int nw = expert ? (cnt + work_rows - 1) / work_rows : 0;
+  const int nw = expert ? (cnt + work_rows - 1) >> work_shift(work_rows) : 0;
   nw_long = cnt > kStreamTT4Rows ? nw : 0;
   nw_short = cnt > kStreamTT4Rows ? 0 : nw;
 }
@@ -316,7 +316,8 @@ __device__ void block_dispatch(int id_in, int n, int E, int tile_rows,
     const int pos = ls->off[id] + rank;
     b.sorted[pos] = tid;
     b.inv[tid] = pos;
-    b.work[work_ints(WR) * (ls->wpos[id] + rank / WR) + 4 + rank % WR] = tid;
+    if (rank % WR < kWorkRows)
+      b.work[kWorkInts * (ls->wpos[id] + rank / WR) + 4 + rank % WR] = tid;
   }
   if (tid < E) {
     b.counts[tid] = cnt;
@@ -324,7 +325,7 @@ __device__ void block_dispatch(int id_in, int n, int E, int tile_rows,
   }
   if (has) b.active[apos] = tid;
   for (int j = 0; j < nw; ++j) {
-    int32_t* w = b.work + work_ints(WR) * (wpos + j);
+    int32_t* w = b.work + kWorkInts * (wpos + j);
     w[0] = tid;
     w[1] = off + j * WR;
     w[2] = min(WR, cnt - j * WR);
@@ -373,14 +374,12 @@ __device__ void wave_dispatch(int id_in, int n, int E, int tile_rows,
     const uint64_t bal = __ballot(on);
     match &= on ? bal : ~bal;
   }
-  constexpr int wr = kWorkRows, ws = 3;                     // (work_rows_for: n > 64 if wide)
-  static_assert(1 << ws == wr, "a shift");
   const int r = __popcll(match & ((1ull << lane) - 1ull));  // rank among equals
   const int c = ok ? __popcll(match) : 0;                   // the expert's rows
   const bool leader = ok && r == 0;
   // long-form items over all experts: the short-form items start after them
   const uint32_t wl_own =
-      leader && c > kStreamTT4Rows ? (uint32_t)((c + wr - 1) >> ws) : 0u;
+      leader && c > kStreamTT4Rows ? (uint32_t)((c + kWorkRows - 1) / kWorkRows) : 0u;
   const int tot_long = (int)readlane_u32(wave_incl_scan(wl_own), 63);
   for (int e = lane; e < E; e += 64) ls->cnt[e] = 0;
   if (leader) ls->cnt[id] = c;
@@ -390,7 +389,7 @@ __device__ void wave_dispatch(int id_in, int n, int E, int tile_rows,
   for (int e0 = 0; e0 < E; e0 += 64) {
     const int e = e0 + lane;
     const int ce = e < E ? ls->cnt[e] : 0;
-    const int nw = (ce + wr - 1) >> ws;
+    const int nw = (ce + kWorkRows - 1) / kWorkRows;
     const int nt = (ce + tile_rows - 1) / tile_rows;
     const bool lng = ce > kStreamTT4Rows;
     const uint32_t pa = (uint32_t)ce | (ce > 0 ? 1u << 8 : 0u) |
@@ -411,10 +410,10 @@ __device__ void wave_dispatch(int id_in, int n, int E, int tile_rows,
       ls->item[e] = first;
       b.active[(xa >> 8) & 0xffu] = e;
       for (int j = 0; j < nw; ++j) {
-        int32_t* w = b.work + work_ints(wr) * (first + j);
+        int32_t* w = b.work + kWorkInts * (first + j);
         w[0] = e;
-        w[1] = off + j * wr;
-        w[2] = min(wr, ce - j * wr);
+        w[1] = off + j * kWorkRows;
+        w[2] = min(kWorkRows, ce - j * kWorkRows);
         w[3] = ce;
       }
       const int tb = (int)((xa >> 16) & 0xffu);
@@ -428,7 +427,7 @@ __device__ void wave_dispatch(int id_in, int n, int E, int tile_rows,
     const int pos = ls->pos[id] + r;
     b.sorted[pos] = lane;
     b.inv[lane] = pos;
-    b.work[work_ints(wr) * (ls->item[id] + (r >> ws)) + 4 + (r & (wr - 1))] = lane;
+    b.work[kWorkInts * (ls->item[id] + r / kWorkRows) + 4 + r % kWorkRows] = lane;
   }
   if (lane == 0) {
     b.offsets[E] = (int)(carry_a & 0xffu);

@@ -97,26 +97,21 @@ def test_noalloc_refuses_oversize_on_host(pkg):
     assert "null module" in C.last_error()
 
 
-def test_noalloc_limit_without_the_wide_records_room(pkg):
-    """The largest T the no-alloc block forward takes is that of the workspace
-    without the room the 16-row items' records need beyond the 8-row ones
-    (a taken call ends here at the device lookup or the null-array check)."""
+@pytest.mark.parametrize("E,K", [(512, 1), (256, 8), (64, 6)])
+def test_noalloc_takes_every_T_that_fits_its_scratch(pkg, E, K):
+    """The no-alloc block forward takes a T exactly when its workspace size is
+    within the library's scratch, as the header says, whatever work items its
+    rows make (16-row ones from 6 rows an expert).  (A taken call ends here at
+    the device lookup or the null-array check.)"""
     import ctypes
-    blk = _tiny_block(pkg, d=512, E=512, K=1)
+    blk = _tiny_block(pkg, d=512, E=E, K=K)
     lib, C = pkg._capi.lib(), pkg._capi
     cap = lib.mlxr_moe_noalloc_scratch_size()
-
-    def room(t):
-        n, E = t, 512
-        a, b = (4 * ints for ints in (12 * (min(E, n) + n // 8), 20 * (min(E, n) + n // 16)))
-        return max(0, -(-b // 256) * 256 - -(-a // 256) * 256)
-
-    lo, hi = 1, 16384
+    lo, hi = 1, 1 << 16
     while hi - lo > 1:
         mid = (lo + hi) // 2
-        lo, hi = (mid, hi) if blk.workspace_size(mid) - room(mid) <= cap else (lo, mid)
-    assert room(lo) > 0 and blk.workspace_size(lo) > cap
-    for t, refused in ((lo, False), (hi, True)):
+        lo, hi = (mid, hi) if blk.workspace_size(mid) <= cap else (lo, mid)
+    for t, refused in ((lo - 1, False), (lo, False), (hi, True), (hi + 1, True)):
         rc = lib.mlxr_moe_block_forward_noalloc(ctypes.byref(blk.descriptor()), None, t,
                                                 None, None, None, None)
         assert rc == -1 and ("bytes of scratch" in C.last_error()) == refused

@@ -69,7 +69,8 @@ __device__ __forceinline__ uint32_t and_opaque(uint32_t x, uint32_t m) {
 // is the f16 subnormal code * 2^-24 (code * 2^-20 four bits up), and
 // v_fma_mix_f32 multiplies it as it is by s * 2^24 (s * 2^20): the product is
 // code * s exactly, so the sum is rounded once, as fmaf(code, s, b) is (for
-// |s| < 2^104, where s * 2^24 is finite).  17 instructions a word against 23
+// |s| < 2^104, where s * 2^24 is finite: a unit with a larger scale is done
+// again by exact4_unit).  17 instructions a word against 23
 // with a v_cvt_f32_ubyte per code: step of c3 T=4096 509 to 502 us, c4 T=2048
 // 489 to 481, bit-identical.
 __device__ __forceinline__ void dequant4(uint32_t w, float s24, float s20, float b,
@@ -87,6 +88,13 @@ __device__ __forceinline__ void dequant4(uint32_t w, float s24, float s20, float
     o[2 * j + 1] = pack_bf16(__builtin_fmaf((float)c26[j], s24, b),
                              __builtin_fmaf((float)c37[j], s20, b));
   }
+}
+// The same words by fmaf(code, s, b) as it stands, for scales of any size.
+__device__ __forceinline__ void dequant4_any(uint32_t w, float s, float b, uint32_t* o) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    o[j] = pack_bf16(__builtin_fmaf((float)((w >> (8 * j)) & 15u), s, b),
+                     __builtin_fmaf((float)((w >> (8 * j + 4)) & 15u), s, b));
 }
 // 4 eight-bit codes -> 2 words of pairs
 __device__ __forceinline__ void dequant8(uint32_t w, float s, float b,

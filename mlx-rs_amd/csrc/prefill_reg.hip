@@ -61,9 +61,10 @@ template <int BITS>
 constexpr int kMacroGroups = BITS == 4 ? 4 : 2;
 
 // The rows [slot0, slot0 + rows) of expert e against N-tiles [nt0, nt1).
-// NMB: 32-row blocks that hold rows.  RES: x whole in LDS.
+// NMB: 32-row blocks that hold rows.  RES: x whole in LDS.  Returns (for the
+// whole wave) whether a 4-bit scale may have been too large (exact4_unit).
 template <int BITS, bool GATED, int SBM, bool RES, int NMB>
-__device__ __forceinline__ void reg_unit(const RegArgs& a, int N, int K, int e, int slot0,
+__device__ __forceinline__ bool reg_unit(const RegArgs& a, int N, int K, int e, int slot0,
                                          int rows, int nt0, int nt1, char* smem) {
   constexpr int SG = kStepGroups<BITS>, MG = kMacroGroups<BITS>;
   constexpr int TC = GATED ? 32 * kWaves : 64 * kWaves;  // channels per N-tile
@@ -378,7 +379,10 @@ __device__ __forceinline__ void reg_unit(const RegArgs& a, int N, int K, int e, 
   // ---- a finished tile: through the wave's scratch, 32 rows at a time, so
   // that every store is 16 bytes of a row
   uint16_t* O = reinterpret_cast<uint16_t*>(scratch);
+  uint64_t nonfinite = 0;  // (a scale too large: not one sum of its channel is finite)
   auto epilogue = [&](int nt) {
+    if constexpr (BITS == 4)
+      nonfinite |= __ballot(!__builtin_isfinite(acc[0][0][0]) || !__builtin_isfinite(acc[0][1][0]));
     const int och0 = nt * TC + wave * WC;
 #pragma unroll
     for (int mb = 0; mb < NMB; ++mb) {
@@ -498,39 +502,26 @@ __device__ __forceinline__ void reg_unit(const RegArgs& a, int N, int K, int e, 
 #pragma nounroll
     for (int q = 0; q < total; ++q) macro(W0, W1);
   }
+  return nonfinite != 0;
 }
 
-// Workgroups go to the XCDs round robin (blockIdx % kXcds).  Each XCD takes an
-// eighth of the M-tile list, in order, a tile's units one after another: they
-// share the tile's x rows, and an expert's further tiles its weights, in that
-// XCD's L2.  (Tiles dealt to the XCDs in turn: c5 T=512 step 679 us against
-// 657, c3 T=512 177 against 168, c4 T=2048 428 against 427; a few tiles'
-// units interleaved: 1-5% slower.)  The folded problem's tiles come first.
 template <int BITS, bool GATED, int SBM, bool RES>
-__global__ __launch_bounds__(kNT, 2) void qgemm_prefill_reg_kernel(
-    QGemmArgs a, int tiles_n, int ntl, int units_n, uint32_t x_bytes, QGemmArgs a2, int tiles2, int rows2, uint32_t x_bytes2) {
+__global__ __launch_bounds__(kNT, 2) void qgemm_prefill_reg_kernel(RegLaunch L) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int grid2 = reg_grid(tiles2, units_n);
-  const bool second = (int)blockIdx.x < grid2;
-  const int b = second ? (int)blockIdx.x : (int)blockIdx.x - grid2;
-  const int xcd = b % (int)kXcds, jx = b / (int)kXcds;
-  const int n_tiles = second ? tiles2 : *a.num_tiles;
-  const int tile = xcd * n_tiles / (int)kXcds + jx / units_n;
-  if (tile >= (xcd + 1) * n_tiles / (int)kXcds) return;
-  const int nt0 = (jx - jx / units_n * units_n) * ntl, nt1 = min(nt0 + ntl, tiles_n);
-  int e = 0, slot0 = tile * kRows, end = rows2;
-  if (!second) {
-    const int2 trec = *reinterpret_cast<const int2*>(a.tiles + 2 * tile);
-    e = __builtin_amdgcn_readfirstlane(trec.x);
-    slot0 = __builtin_amdgcn_readfirstlane(trec.y);
-    end = __builtin_amdgcn_readfirstlane(a.offsets[e + 1]);
-  }
-  const int rows = min(kRows, end - slot0);
-  const RegArgs r = pick_reg(second, a2, x_bytes2, a, x_bytes);
-  if (rows > 32)
-    reg_unit<BITS, GATED, SBM, RES, 2>(r, a.N, a.K, e, slot0, rows, nt0, nt1, smem);
+  RegUnit<kRows> u;
+  if (!u.place(L, blockIdx.x)) return;
+  u.find_rows(L);
+  const RegArgs r = pick_reg(u.second, L.a2, L.x_bytes2, L.a, L.x_bytes);
+  bool nonfinite;
+  if (u.rows > 32)
+    nonfinite = reg_unit<BITS, GATED, SBM, RES, 2>(r, L.a.N, L.a.K, u.e, u.slot0, u.rows,
+                                                  u.nt0, u.nt1, smem);
   else
-    reg_unit<BITS, GATED, SBM, RES, 1>(r, a.N, a.K, e, slot0, rows, nt0, nt1, smem);
+    nonfinite = reg_unit<BITS, GATED, SBM, RES, 1>(r, L.a.N, L.a.K, u.e, u.slot0, u.rows,
+                                                  u.nt0, u.nt1, smem);
+  if constexpr (BITS == 4) {
+    if (nonfinite) exact4_unit<GATED, kRows>(kWaves);
+  }
 }
 
 }  // namespace
@@ -566,12 +557,11 @@ hipError_t launch_qgemm_prefill_reg(const QGemmArgs& a, int64_t x_rows, int64_t 
                                   : G % 2 == 0 && (sb_addr & 3) == 0;
   const bool res = G <= kResGroups;
   const dim3 grid((unsigned)(reg_grid(max_tiles, units_n) + reg_grid(tiles2, units_n)));
-  const uint32_t x_bytes = (uint32_t)(x_rows * a.x_ld * 2);
-  const uint32_t x_bytes2 = (uint32_t)(rows2 * b.x_ld * 2);
+  const RegLaunch L{a, tiles_n, ntl, units_n, (uint32_t)(x_rows * a.x_ld * 2),
+                    b, (int32_t)tiles2, (int32_t)rows2, (uint32_t)(rows2 * b.x_ld * 2)};
   ProfileScope prof(profile, s);
 #define MLXR_PR(B, G_, V, R)                                                               \
-  qgemm_prefill_reg_kernel<B, G_, V, R><<<grid, kNT, reg_lds(V, R), s>>>(                  \
-      a, tiles_n, ntl, units_n, x_bytes, b, (int)tiles2, (int)rows2, x_bytes2)
+  qgemm_prefill_reg_kernel<B, G_, V, R><<<grid, kNT, reg_lds(V, R), s>>>(L)
   // (a gated launch of K <= 512 takes the general form: one instance less)
 #define MLXR_PR_V(B, V)            \
   do {                             \

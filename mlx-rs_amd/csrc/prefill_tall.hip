@@ -46,9 +46,10 @@ constexpr int tall_lds(int sbm) {
 static_assert(2 * tall_lds(kSbLds) <= 160 * 1024, "two workgroups per CU");
 
 // The rows [slot0, slot0 + rows) of expert e against N-tiles [nt0, nt1).
-// NMB: 32-row blocks that hold rows.
+// NMB: 32-row blocks that hold rows.  Returns (for the whole wave) whether a
+// 4-bit scale may have been too large (exact4_unit).
 template <int BITS, bool GATED, int SBM, int NMB>
-__device__ __forceinline__ void tall_unit(const RegArgs& a, int N, int K, int e, int slot0,
+__device__ __forceinline__ bool tall_unit(const RegArgs& a, int N, int K, int e, int slot0,
                                          int rows, int nt0, int nt1, char* smem) {
   constexpr int SG = kStepGroups<BITS>;  // groups per weight step
   constexpr int TC = GATED ? 32 * kWaves : 64 * kWaves;  // channels per N-tile
@@ -334,7 +335,10 @@ __device__ __forceinline__ void tall_unit(const RegArgs& a, int N, int K, int e,
   // ---- a finished tile: through the wave's scratch, 32 rows at a time, so
   // that every store is 16 bytes of a row
   uint16_t* O = reinterpret_cast<uint16_t*>(scratch);
+  uint64_t nonfinite = 0;  // (a scale too large: not one sum of its channel is finite)
   auto epilogue = [&](int nt) {
+    if constexpr (BITS == 4)
+      nonfinite |= __ballot(!__builtin_isfinite(acc[0][0][0]) || !__builtin_isfinite(acc[0][1][0]));
     const int och0 = nt * TC + wave * WC;
     // (the lane anew, so that what the stores make of it is made here: kept
     // over the weight steps it was ten registers too many)
@@ -463,39 +467,32 @@ __device__ __forceinline__ void tall_unit(const RegArgs& a, int N, int K, int e,
       ++nt;
     }
   }
+  return nonfinite != 0;
 }
 
-// Workgroup numbering: as prefill_reg.hip.
 template <int BITS, bool GATED, int SBM>
-__global__ __launch_bounds__(kNT, 2) void qgemm_prefill_tall_kernel(
-    QGemmArgs a, int tiles_n, int ntl, int units_n, uint32_t x_bytes, QGemmArgs a2,
-    int tiles2, int rows2, uint32_t x_bytes2) {
+__global__ __launch_bounds__(kNT, 2) void qgemm_prefill_tall_kernel(RegLaunch L) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int grid2 = reg_grid(tiles2, units_n);
-  const bool second = (int)blockIdx.x < grid2;
-  const int b = second ? (int)blockIdx.x : (int)blockIdx.x - grid2;
-  const int xcd = b % (int)kXcds, jx = b / (int)kXcds;
-  const int n_tiles = second ? tiles2 : *a.num_tiles;
-  const int tile = xcd * n_tiles / (int)kXcds + jx / units_n;
-  if (tile >= (xcd + 1) * n_tiles / (int)kXcds) return;
-  const int nt0 = (jx - jx / units_n * units_n) * ntl, nt1 = min(nt0 + ntl, tiles_n);
-  int e = 0, slot0 = tile * kRows, end = rows2;
-  if (!second) {
-    const int2 trec = *reinterpret_cast<const int2*>(a.tiles + 2 * tile);
-    e = __builtin_amdgcn_readfirstlane(trec.x);
-    slot0 = __builtin_amdgcn_readfirstlane(trec.y);
-    end = __builtin_amdgcn_readfirstlane(a.offsets[e + 1]);
-  }
-  const int rows = min(kRows, end - slot0);
-  const RegArgs r = pick_reg(second, a2, x_bytes2, a, x_bytes);
-  if (rows > 96)
-    tall_unit<BITS, GATED, SBM, 4>(r, a.N, a.K, e, slot0, rows, nt0, nt1, smem);
-  else if (rows > 64)
-    tall_unit<BITS, GATED, SBM, 3>(r, a.N, a.K, e, slot0, rows, nt0, nt1, smem);
-  else if (rows > 32)
-    tall_unit<BITS, GATED, SBM, 2>(r, a.N, a.K, e, slot0, rows, nt0, nt1, smem);
+  RegUnit<kRows> u;
+  if (!u.place(L, blockIdx.x)) return;
+  u.find_rows(L);
+  const RegArgs r = pick_reg(u.second, L.a2, L.x_bytes2, L.a, L.x_bytes);
+  bool nonfinite;
+  if (u.rows > 96)
+    nonfinite = tall_unit<BITS, GATED, SBM, 4>(r, L.a.N, L.a.K, u.e, u.slot0, u.rows, u.nt0,
+                                              u.nt1, smem);
+  else if (u.rows > 64)
+    nonfinite = tall_unit<BITS, GATED, SBM, 3>(r, L.a.N, L.a.K, u.e, u.slot0, u.rows, u.nt0,
+                                              u.nt1, smem);
+  else if (u.rows > 32)
+    nonfinite = tall_unit<BITS, GATED, SBM, 2>(r, L.a.N, L.a.K, u.e, u.slot0, u.rows, u.nt0,
+                                              u.nt1, smem);
   else
-    tall_unit<BITS, GATED, SBM, 1>(r, a.N, a.K, e, slot0, rows, nt0, nt1, smem);
+    nonfinite = tall_unit<BITS, GATED, SBM, 1>(r, L.a.N, L.a.K, u.e, u.slot0, u.rows, u.nt0,
+                                              u.nt1, smem);
+  if constexpr (BITS == 4) {
+    if (nonfinite) exact4_unit<GATED, kRows>(kWaves);
+  }
 }
 
 }  // namespace
@@ -528,12 +525,11 @@ hipError_t launch_qgemm_prefill_tall(const QGemmArgs& a, int64_t x_rows, int64_t
   const bool sb_vec = a.bits == 4 ? G % 4 == 0 && (sb_addr & 7) == 0
                                   : G % 2 == 0 && (sb_addr & 3) == 0;
   const dim3 grid((unsigned)(reg_grid(max_tiles, units_n) + reg_grid(tiles2, units_n)));
-  const uint32_t x_bytes = (uint32_t)(x_rows * a.x_ld * 2);
-  const uint32_t x_bytes2 = (uint32_t)(rows2 * b.x_ld * 2);
+  const RegLaunch L{a, tiles_n, ntl, units_n, (uint32_t)(x_rows * a.x_ld * 2),
+                    b, (int32_t)tiles2, (int32_t)rows2, (uint32_t)(rows2 * b.x_ld * 2)};
   ProfileScope prof(profile, s);
 #define MLXR_PT(B, G_, V)                                                        \
-  qgemm_prefill_tall_kernel<B, G_, V><<<grid, kNT, tall_lds(V), s>>>(            \
-      a, tiles_n, ntl, units_n, x_bytes, b, (int)tiles2, (int)rows2, x_bytes2)
+  qgemm_prefill_tall_kernel<B, G_, V><<<grid, kNT, tall_lds(V), s>>>(L)
 #define MLXR_PT_V(B, V)       \
   do {                        \
     if (a.gated)              \

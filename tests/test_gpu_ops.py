@@ -400,6 +400,60 @@ def test_gather_qmm_register_tiles(pkg, dev, bits, N, K, offset, counts):
         assert bool(((got[r, 0].double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("counts", [SHORT_COUNTS, TALL_COUNTS], ids=["short", "tall"])
+@pytest.mark.parametrize("f,d,offset", [(64, 512, 0), (320, 768, 0), (128, 2048, 0), (192, 576, 0),
+                                        (192, 512, 1)])
+def test_tiled_qmm_scales_up_to_the_top_of_the_range(pkg, dev, f, d, offset, counts):
+    """4-bit scales of 2^104 and more, on a few channels of some experts: the
+    tiled kernels' scaled forms of a scale overflow there.  Equal to the dense
+    kernels on the dequantised weights, as an op and as a gated FFN (SwiGLU and
+    packed GeGLU), and finite."""
+    E, B = len(counts), sum(counts)
+    assert pkg.ops.gather_qmm_tiled(B, E)
+    g = torch.Generator(device=dev)
+    g.manual_seed(d + f)
+    ids = torch.repeat_interleave(torch.arange(E, device=dev), torch.tensor(counts, device=dev))
+    ids = ids[torch.randperm(B, generator=g, device=dev)].to(torch.int32)
+
+    def at(v):
+        buf = torch.zeros(v.numel() + offset, dtype=v.dtype, device=dev)
+        buf[offset:] = v.reshape(-1)
+        return buf[offset:].view(v.shape)
+
+    def bank(n, k, low, high):
+        wq = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, n, k // 8), generator=g, device=dev,
+                           dtype=torch.int64).to(torch.int32)
+        p = torch.full((E, n, k // 64), low, device=dev)
+        p[::3, ::37, -1] = high
+        p[1::3, 5::41, 0] = high + 1
+        sc, bi = ((1 + torch.rand(p.shape, generator=g, device=dev)) * 2.0 ** p for _ in range(2))
+        q = (wq, at(sc.to(torch.bfloat16)), at((-7 * bi).to(torch.bfloat16)))
+        return q, pkg.ops.dequantize(*q, 64, 4)
+
+    # values of about 1 and below from weights of up to 2^124: x is tiny
+    x = (torch.randn((B, d), generator=g, device=dev) * 2.0 ** -115).to(torch.bfloat16)
+    gate, up = bank(f, d, 100.0, 119.0), bank(f, d, 104.0, 110.0)
+    for q, w in (gate, up):
+        assert bool(w.isfinite().all()) and float(w.abs().max()) > 2.0 ** 112
+        got = pkg.ops.gather_qmm(x[:, None], *q, None, ids, True, 64, 4)
+        assert bool(got.isfinite().all())
+        assert torch.equal(got, pkg.ops.gather_mm(x[:, None], w, None, ids))
+    down = bank(d, f, -4.0, 105.0)
+    nn = pkg.nn
+    quant, dense = [], []
+    for q, w in (gate, up, down):
+        quant.append(nn.QuantizedSwitchLinear(*q, 64, 4))
+        dense.append(nn.SwitchLinear(w))
+    got, want = (nn.SplitSwitchFfn(*m).forward(x, ids[:, None]) for m in (quant, dense))
+    assert bool(got.isfinite().all()) and torch.equal(got, want)
+    pq = tuple(torch.cat((a, b), 1) for a, b in zip(gate[0], up[0]))
+    pw = torch.cat((gate[1], up[1]), 1)
+    got, want = (nn.PackedSwitchFfn(m, n, "geglu").forward(x, ids[:, None])
+                 for m, n in ((nn.QuantizedSwitchLinear(*pq, 64, 4), quant[2]),
+                              (nn.SwitchLinear(pw), dense[2])))
+    assert bool(got.isfinite().all()) and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("E,N,K", [
     (64, 128, 256), (64, 64, 512), (64, 128, 768), (64, 192, 1536), (64, 128, 2048),

@@ -210,7 +210,7 @@ struct QGemmArgs {
   const int32_t* row_map;
   int32_t row_div;
   bool x_by_slot;
-  uint8_t work_rows;       // rows per work item (the launcher's; in padding)
+  uint8_t work_rows;       // rows per work item (in what would be padding)
   const int32_t* offsets;  // [E+1] slot range of each expert
   const int32_t* active;   // [E] experts with rows
   const int32_t* num_active;
@@ -237,12 +237,13 @@ struct QGemmArgs {
 // one in seven experts has over kWorkRows rows: at 6 rows per expert a step of
 // c2 (T = 96) went from 117 us to 114, c6 (T = 200) 193 to 188; with fewer, the
 // 8-row items' kernel covers nearly every expert in one item and has the
-// smaller LDS and register footprint.  Only where every GEMM runs the streaming
-// kernel, without K-slices, with 8-row items: then the sums are those of 8-row
-// items, and the grid is large enough for items twice as long (a one-expert
-// MLP of d 2048, f 512 at T = 200 took 35.4 us in wide items, 33.3 in K-sliced
-// 8-row ones).  Input dims that the wide form stages (stream16_body); more
-// than 64 rows (the one-wave sort of fewer makes 8-row items).
+// smaller LDS and register footprint.  Only for grids of kStreamMinBlocks units
+// and more, and not where 8-row items would run the streaming kernel in
+// K-slices: then every sum is that of 8-row items, and the grid is large enough
+// for items twice as long (a one-expert MLP of d 2048, f 512 at T = 200 took
+// 35.4 us in wide items, 33.3 in K-sliced 8-row ones).  Input dims that the wide
+// form stages (stream16_body); more than 64 rows (the one-wave sort of fewer
+// makes 8-row items).
 #ifndef MLXR_WIDE_ITEM_ROWS
 #define MLXR_WIDE_ITEM_ROWS 6
 #endif

@@ -175,10 +175,11 @@ __device__ __forceinline__ void decode_body(const QGemmArgs& a, int tile,
     int64_t xrow = 0;
     if (tv) {
       const int slot = row0 + tok;
-      // this lane's flat row from the record (tok < kWorkRows = 8)
+      // this lane's flat row from the record (its first eight fetched with the
+      // header; a wide item's others from the sorted list)
       const int f4 = (tok & 3) == 0 ? fr0.x : (tok & 3) == 1 ? fr0.y : (tok & 3) == 2 ? fr0.z : fr0.w;
       const int f8 = (tok & 3) == 0 ? fr1.x : (tok & 3) == 1 ? fr1.y : (tok & 3) == 2 ? fr1.z : fr1.w;
-      const int flat = tok < 4 ? f4 : f8;
+      const int flat = tok < 4 ? f4 : tok < kWorkRows ? f8 : a.x_by_slot ? 0 : a.sorted[slot];
       xrow = a.x_by_slot ? slot : (a.row_map ? a.row_map[flat] : flat / a.row_div);
     }
     f32x4_t acc[CB][NM];
@@ -315,7 +316,8 @@ __device__ __forceinline__ void decode_body(const QGemmArgs& a, int tile,
             a.out[(int64_t)slot * a.out_ld + ch] =
                 gated_act_bf16(a.act, bf16_round(s0[r]), bf16_round(s1[r]));
           } else {
-            const int64_t orow = a.out_by_flat ? rec[4 + t] : slot;
+            const int64_t orow =
+                !a.out_by_flat ? slot : t < kWorkRows ? rec[4 + t] : a.sorted[slot];
             a.out[orow * a.out_ld + ch] = f32_to_bf16(s0[r]);
           }
         }
@@ -329,7 +331,7 @@ template <int BITS, bool GATED, int SPW, int CB>
 __global__ __launch_bounds__(1024) void qgemm_decode_kernel(
     QGemmArgs a, int tiles_n, QGemmArgs a2, int units1, int items1, int rows2) {
   Unit u;
-  if (!decode_unit(a, tiles_n, units1, items1, rows2, u)) return;
+  if (!decode_unit<0>(a, tiles_n, units1, items1, rows2, u)) return;
   decode_body<BITS, GATED, SPW, CB>(u.shared ? a2 : a, u.tile, u.rec, u.wk,
                                     u.fr0, u.fr1);
 }
@@ -527,11 +529,15 @@ StreamShape stream_shape(const QGemmArgs& a, int64_t all_items) {
 
 int work_rows_for(int64_t n, int64_t E, std::initializer_list<const QGemmArgs*> gemms) {
   if (n <= 64 || n < MLXR_WIDE_ITEM_ROWS * E) return kWorkRows;
-  for (const QGemmArgs* g : gemms)
-    if (!(g->K <= kWideWhole || g->K % kWideSlice == 0) ||
-        !stream_eligible(*g, *g, dispatch_max_work(n, E, kWorkRowsWide)) ||
+  const int64_t items = dispatch_max_work(n, E, kWorkRowsWide);
+  for (const QGemmArgs* g : gemms) {
+    if (g->bits == 16 || !(g->K <= kWideWhole || g->K % kWideSlice == 0) ||
+        items * (g->N / 16) < kStreamMinBlocks)
+      return kWorkRows;
+    if (stream_eligible(*g, *g, items) &&
         stream_shape(*g, dispatch_max_work(n, E, kWorkRows)).ks > 1)
       return kWorkRows;
+  }
   return kWorkRowsWide;
 }
 
@@ -564,9 +570,9 @@ hipError_t launch_qgemm(const QGemmArgs& a, int64_t total_rows,
   // spreads each block over up to 16 waves.
   const int64_t all_items = max_items + items2;
   // (dense bf16 weights, bits 16, take the split-K kernel below)
-  if (a.work_rows == kWorkRowsWide)
-    return launch_stream_wide(a, b, max_items, items2, shared_rows, profile, s);
   if (stream_eligible(a, b, all_items)) {
+    if (a.work_rows == kWorkRowsWide)
+      return launch_stream_wide(a, b, max_items, items2, shared_rows, profile, s);
     constexpr int kWaves = MLXR_STREAM_WAVES;
     const StreamShape sh = stream_shape(a, all_items);
     const int nb = sh.nb, ks = sh.ks, tiles_n = sh.tiles_n;

@@ -140,7 +140,7 @@ struct Unit {
   int tile;
   bool shared;
 };
-template <int WR = kWorkRows>  // rows per item
+template <int WR = kWorkRows>  // rows per item, or 0: a.work_rows
 __device__ __forceinline__ bool decode_unit(const QGemmArgs& a, int tiles_n,
                                             int units1, int items1, int rows2,
                                             Unit& u) {
@@ -150,14 +150,15 @@ __device__ __forceinline__ bool decode_unit(const QGemmArgs& a, int tiles_n,
   u.tile = v - ai * tiles_n;
   // (the routed record is read unconditionally, item 0's for a shared
   // unit)
+  const int wr = WR ? WR : a.work_rows;
   u.rec = a.work + (int64_t)kWorkInts * (u.shared ? 0 : min(ai, items1 - 1));
   u.wk = *reinterpret_cast<const int4*>(u.rec);
   u.fr0 = *reinterpret_cast<const int4*>(u.rec + 4);
   u.fr1 = *reinterpret_cast<const int4*>(u.rec + 8);
   const int n_act = *a.num_work;
   if (u.shared) {
-    const int r0 = WR * ai;
-    u.wk = make_int4(0, r0, min(WR, rows2 - r0), rows2);
+    const int r0 = wr * ai;
+    u.wk = make_int4(0, r0, min(wr, rows2 - r0), rows2);
     u.fr0 = make_int4(r0, r0 + 1, r0 + 2, r0 + 3);
     u.fr1 = make_int4(r0 + 4, r0 + 5, r0 + 6, r0 + 7);
     return true;

@@ -495,11 +495,11 @@ def test_gather_qmm_wide_items(pkg, dev, bits, E, N, K):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("d", [256, 768, 1536, 2048, 4096])
+@pytest.mark.parametrize("d", [256, 320, 768, 1536, 2048, 4096])
 def test_wide_items_sum_as_eight_row_items(pkg, dev, bits, d):
     """A row's result does not depend on the item it runs in: experts of 9 to 33
     rows in one call (16-row items, x staged whole and in slices), and the same
-    rows eight an expert at a time (the 8-token form).  Equal bits, for one
+    rows eight an expert at a time (8-token form; d = 320: split-K).  Equal bits, for one
     projection as an op and for the gated FFN."""
     E, f = 64, 256
     counts = [16, 17, 9, 12, 33, 9, 10, 9] * (E // 8)

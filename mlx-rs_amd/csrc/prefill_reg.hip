@@ -124,17 +124,15 @@ __device__ __forceinline__ bool reg_unit(const RegArgs& a, int N, int K, int e, 
         const uint16_t* bp = GATED && s ? a.w1.biases : a.w0.biases;
         const int ch = min(channel0(on ? pt : nt0, s) + c, N - 1);
         const gptr<const uint16_t> p =
-            as_global<const uint16_t>(h ? bp : sp) + ((int64_t)e * a.e_rows + ch) * G + g0;
-        W.sb[s][0] = W.sb[s][1] = 0u;
+            as_global<const uint16_t>(h ? bp : sp) + (int64_t)e * a.e_rows * G;
         if constexpr (SBM == kSbVector && BITS == 4) {
-          const u32x2_t v = *(gptr<const u32x2_t>)p;
+          const u32x2_t v = *(gptr<const u32x2_t>)(p + (int64_t)ch * G + g0);
           W.sb[s][0] = v.x, W.sb[s][1] = v.y;
         } else if constexpr (SBM == kSbVector) {
-          W.sb[s][0] = *(gptr<const uint32_t>)p;
+          W.sb[s][0] = *(gptr<const uint32_t>)(p + (int64_t)ch * G + g0);
+          W.sb[s][1] = 0u;
         } else {
-#pragma unroll
-          for (int j = 0; j < SG; ++j)
-            W.sb[s][j / 2] |= (uint32_t)p[min(j, G - 1 - g0)] << (16 * (j & 1));
+          load_sb_any<SG>(p, N, G, ch, g0, W.sb[s]);
         }
       }
     }
@@ -214,7 +212,8 @@ __device__ __forceinline__ bool reg_unit(const RegArgs& a, int N, int K, int e, 
   }
   const int aw = (xc >> 3) * kGroupBytes + xrow0 * 128 + 16 * ((xc & 7) ^ swz(xrow0));
   u32x4_t xv[XC];
-  const int XS = S * (MG / 2);  // x stages per tile
+  // x stages per tile: two groups each (rows of kSbAny: up to K's end)
+  const int XS = BITS == 4 && SBM == kSbAny ? (G + 1) / 2 : S * (MG / 2);
   int px = 0, left_x = XS * (nt1 - nt0);
   auto load_x = [&]() {  // the next x stage (zeros past K and past the unit)
     const bool ok = left_x > 0 && 128 * px + 8 * xc < K;
@@ -466,8 +465,9 @@ __device__ __forceinline__ bool reg_unit(const RegArgs& a, int N, int K, int e, 
           store_x(xst ^ 1);
           __syncthreads();
           xst ^= 1;
-          if (gi + 2 < SG) load_x();
         }
+        if (BITS == 4 && SBM == kSbAny && SG * s + gi + 2 >= G) break;  // K's end
+        if (!RES && gi + 2 < SG) load_x();
       }
       if constexpr (SBM == kSbLds) {
         if (g32 >= min(kSbChunk, G - kSbChunk * ck)) {
@@ -579,10 +579,10 @@ hipError_t launch_qgemm_prefill_reg(const QGemmArgs& a, int64_t x_rows, int64_t 
     else if (sb_vec)            \
       MLXR_PR_V(B, kSbVector);  \
     else                        \
-      MLXR_PR_V(B, kSbSingle);  \
+      MLXR_PR_V(B, kSbAny);  \
   } while (0)
   if (a.bits == 16)
-    MLXR_PR_V(16, kSbSingle);
+    MLXR_PR_V(16, kSbAny);
   else if (a.bits == 4)
     MLXR_PR_S(4);
   else

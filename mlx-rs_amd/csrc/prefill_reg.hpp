@@ -10,9 +10,9 @@ namespace mlxr_moe {
 
 constexpr uint32_t kPastEnd = 0xFFFFFFF0u;  // out of range of every buffer
 
-// Where the scales and biases of a weight step come from: single loads, one
-// aligned vector per row, or chunks of several steps in LDS.
-enum { kSbSingle, kSbVector, kSbLds };
+// Where the scales and biases of a weight step come from: rows of any length at
+// any alignment, one aligned vector per row, or chunks of several steps in LDS.
+enum { kSbAny, kSbVector, kSbLds };
 
 // Workgroups of a problem of at most `tiles` M-tiles.
 __host__ __device__ constexpr int reg_grid(int64_t tiles, int units_n) {
@@ -135,6 +135,30 @@ using gptr = __attribute__((address_space(1))) T*;
 template <class T>
 __device__ __forceinline__ gptr<T> as_global(const void* p) {
   return (gptr<T>)reinterpret_cast<uintptr_t>(p);
+}
+
+// The scales (or biases) of a step of SG groups from g0 on, of row ch of an
+// expert's N rows of G, two to a word; zeros past the row, so that a step's
+// groups past it add nothing, whatever the row holds.  One load that needs no
+// more than the elements' alignment, ending within the expert's rows (the rest
+// is shifted out), and no branch around it: that would make the compiler wait
+// for every load in flight.
+template <int SG>
+__device__ __forceinline__ void load_sb_any(gptr<const uint16_t> expert, int N, int G, int ch,
+                                            int g0, uint32_t (&sb)[2]) {
+  typedef uint64_t u64_a2 __attribute__((aligned(2)));
+  typedef uint32_t u32_a2 __attribute__((aligned(2)));
+  const uint32_t off = (uint32_t)(ch * G + g0), at = min(off, (uint32_t)(N * G - SG));
+  const uint32_t sh = 16 * (off - at);
+  const int left = G - g0;
+  if constexpr (SG == 4) {
+    const uint64_t mask = left < 4 ? (1ull << (16 * left)) - 1 : ~0ull;
+    const uint64_t v = (*(gptr<const u64_a2>)(expert + at) >> sh) & mask;
+    sb[0] = (uint32_t)v, sb[1] = (uint32_t)(v >> 32);
+  } else {
+    sb[0] = (*(gptr<const u32_a2>)(expert + at) >> sh) & (left < 2 ? 0xffffu : ~0u);
+    sb[1] = 0u;
+  }
 }
 
 // Wave-private LDS hand-over.

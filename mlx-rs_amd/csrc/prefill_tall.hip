@@ -108,17 +108,15 @@ __device__ __forceinline__ bool tall_unit(const RegArgs& a, int N, int K, int e,
         const uint16_t* bp = GATED && s ? a.w1.biases : a.w0.biases;
         const int ch = min(channel0(on ? pt : nt0, s) + c, N - 1);
         const gptr<const uint16_t> p =
-            as_global<const uint16_t>(h ? bp : sp) + ((int64_t)e * a.e_rows + ch) * G + g0;
-        W.sb[s][0] = W.sb[s][1] = 0u;
+            as_global<const uint16_t>(h ? bp : sp) + (int64_t)e * a.e_rows * G;
         if constexpr (SBM == kSbVector && BITS == 4) {
-          const u32x2_t v = *(gptr<const u32x2_t>)p;
+          const u32x2_t v = *(gptr<const u32x2_t>)(p + (int64_t)ch * G + g0);
           W.sb[s][0] = v.x, W.sb[s][1] = v.y;
         } else if constexpr (SBM == kSbVector) {
-          W.sb[s][0] = *(gptr<const uint32_t>)p;
+          W.sb[s][0] = *(gptr<const uint32_t>)(p + (int64_t)ch * G + g0);
+          W.sb[s][1] = 0u;
         } else {
-#pragma unroll
-          for (int j = 0; j < SG; ++j)
-            W.sb[s][j / 2] |= (uint32_t)p[min(j, G - 1 - g0)] << (16 * (j & 1));
+          load_sb_any<SG>(p, N, G, ch, g0, W.sb[s]);
         }
       }
     }
@@ -544,7 +542,7 @@ hipError_t launch_qgemm_prefill_tall(const QGemmArgs& a, int64_t x_rows, int64_t
     else if (sb_vec)            \
       MLXR_PT_V(B, kSbVector);  \
     else                        \
-      MLXR_PT_V(B, kSbSingle);  \
+      MLXR_PT_V(B, kSbAny);  \
   } while (0)
   if (a.bits == 4)
     MLXR_PT_S(4);

@@ -454,6 +454,31 @@ def test_tiled_qmm_scales_up_to_the_top_of_the_range(pkg, dev, f, d, offset, cou
     assert bool(got.isfinite().all()) and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("counts", [SHORT_COUNTS, TALL_COUNTS], ids=["short", "tall"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("K", [64, 128, 192, 320, 448, 576, 1088, 1152, 2112])
+def test_tiled_qmm_infinite_bias_in_the_last_group(pkg, dev, bits, K, counts):
+    """Input dims that end within a step of the tiled kernels' loads: what pads
+    the step must add nothing even where the last group's bias is infinite
+    (0 * inf would make the row's result, +-inf, a NaN)."""
+    E, B, N = len(counts), sum(counts), 192
+    g = torch.Generator(device=dev)
+    g.manual_seed(K + bits)
+    ids = torch.repeat_interleave(torch.arange(E, device=dev), torch.tensor(counts, device=dev))
+    ids = ids[torch.randperm(B, generator=g, device=dev)].to(torch.int32)
+    x = (torch.rand((B, 1, K), generator=g, device=dev) + 0.5).to(torch.bfloat16)
+    wq = torch.randint(-2 ** 31, 2 ** 31 - 1, (E, N, K * bits // 32), generator=g, device=dev,
+                       dtype=torch.int64).to(torch.int32)
+    sc = (torch.rand((E, N, K // 64), generator=g, device=dev) + 0.5).to(torch.bfloat16)
+    bi = -sc
+    bi[:, ::5, -1] = torch.inf
+    bi[:, 1::5, -1] = -torch.inf
+    got = pkg.ops.gather_qmm(x, wq, sc, bi, None, ids, True, 64, bits)
+    assert torch.equal(got, pkg.ops.gather_mm(x, pkg.ops.dequantize(wq, sc, bi, 64, bits),
+                                              None, ids))
+    assert bool((got[:, 0, ::5] == torch.inf).all() and (got[:, 0, 1::5] == -torch.inf).all())
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("E,N,K", [
     (64, 128, 256), (64, 64, 512), (64, 128, 768), (64, 192, 1536), (64, 128, 2048),

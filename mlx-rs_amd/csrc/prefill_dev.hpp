@@ -19,8 +19,6 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   return __builtin_bit_cast(uint32_t,
                             __builtin_convertvector((f32x2_t){lo, hi}, bf16x2_t));
 }
-// f rounded to bf16 (the hardware conversion: round to nearest even)
-__device__ __forceinline__ float bf16_hw(float f) { return (float)(__bf16)f; }
 // a and b rounded to bf16 by one conversion (round to nearest even), as f32
 __device__ __forceinline__ f32x2_t bf16_hw2(float a, float b) {
   const uint32_t p =
@@ -47,13 +45,15 @@ template <bool B>
 struct PfFlag {
   static constexpr bool value = B;
 };
-// q = n / d for 0 <= n < 2^31, 1 <= d <= 2^16: a float estimate and one
-// correction step either way
-__device__ __forceinline__ int div_small(int n, int d, float rd) {
-  int q = (int)((float)n * rd);
-  q -= (q * d > n) ? 1 : 0;
-  q += ((q + 1) * d <= n) ? 1 : 0;
-  return q;
+// n / d for 0 <= n < 2^31, 1 <= d <= 2^16, rd = 1.0f / d: a float estimate
+// (off by up to 3 * 2^-24 of the quotient and one, as many as 385), another of
+// what it leaves (off by one at most), and a correction either way.
+__host__ __device__ __forceinline__ int div_small(int n, int d, float rd) {
+  uint32_t q = (uint32_t)((float)n * rd);
+  int r = (int)((uint32_t)n - q * (uint32_t)d);
+  q += (uint32_t)(int)((float)r * rd);
+  r = (int)((uint32_t)n - q * (uint32_t)d);
+  return (int)q - (r < 0 ? 1 : 0) + (r >= d ? 1 : 0);
 }
 
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));

@@ -1,6 +1,9 @@
 """Host-side argument checks of the Python mirrors: shapes, dtypes and
 devices are rejected before any pointer reaches the C ABI (no GPU needed:
 every case here fails before a kernel could run)."""
+import os
+from pathlib import Path
+
 import pytest
 import torch
 
@@ -115,6 +118,44 @@ def test_noalloc_takes_every_T_that_fits_its_scratch(pkg, E, K):
         rc = lib.mlxr_moe_block_forward_noalloc(ctypes.byref(blk.descriptor()), None, t,
                                                 None, None, None, None)
         assert rc == -1 and ("bytes of scratch" in C.last_error()) == refused
+
+
+def test_div_small_is_exact(tmp_path):
+    """The tiled kernels' row division (flat row / rows per token), compiled for
+    the host: quotients up to 2^31 - 1, around every multiple that a float
+    estimate can miss."""
+    import subprocess
+    src = Path(__file__).resolve().parent.parent / "mlx-rs_amd" / "csrc"
+    (tmp_path / "d.hip").write_text("""
+#include "prefill_dev.hpp"
+#include <cstdio>
+#include <initializer_list>
+int main() {
+  long bad = 0, seen = 0;
+  auto check = [&](long n, int d) {
+    if (n < 0 || n > 2147483647L) return;
+    ++seen;
+    if (mlxr_moe::div_small((int)n, d, 1.0f / (float)d) != (int)(n / d) && bad++ < 5)
+      std::printf("%ld / %d\\n", n, d);
+  };
+  for (int d : {1, 2, 3, 5, 6, 7, 8, 10, 11, 13, 64, 127, 1000, 1023, 4096, 65535, 65536}) {
+    const long top = 2147483647L / d;
+    for (long q = 0; q <= top; q += 1 + top / 40009)
+      for (long k : {-1L, 0L, 1L, d - 1L}) check(q * d + k, d);
+    for (long k = 0; k < 2000; ++k) check(2147483647L - k, d), check(k, d);
+  }
+  check(116867687, 7);
+  std::printf("seen %ld bad %ld\\n", seen, bad);
+  return bad != 0;
+}
+""")
+    exe = tmp_path / "d"
+    subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "-x", "hip", "-O1", "-std=c++17",
+                    "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "-w", "-I", str(src), str(tmp_path / "d.hip"), "-o",
+                    str(exe)], check=True, capture_output=True)
+    res = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout
 
 
 @pytest.mark.parametrize("key", ["c3", "c5"])

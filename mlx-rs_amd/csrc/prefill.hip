@@ -40,12 +40,10 @@ namespace tile256 {
 #define MLXR_PF_TILE_ROWS 256
 #define MLXR_PF_MBLOCKS 4
 #define MLXR_PF_WAVES_N 4
-#define MLXR_PF_REGBUF 2
 #include "prefill_tile.inc"
 #undef MLXR_PF_TILE_ROWS
 #undef MLXR_PF_MBLOCKS
 #undef MLXR_PF_WAVES_N
-#undef MLXR_PF_REGBUF
 }  // namespace tile256
 // 128 rows of dense bf16 weights: 128 columns, 4 waves of 64 x 64, two stages
 // in 64 KB of LDS, so that two workgroups share a CU and one's barrier waits
@@ -55,14 +53,10 @@ namespace tile128n {
 #define MLXR_PF_TILE_ROWS 128
 #define MLXR_PF_MBLOCKS 2
 #define MLXR_PF_WAVES_N 2
-#define MLXR_PF_REGBUF 2
-#define MLXR_PF_STAGES 2
 #include "prefill_tile.inc"
-#undef MLXR_PF_STAGES
 #undef MLXR_PF_TILE_ROWS
 #undef MLXR_PF_MBLOCKS
 #undef MLXR_PF_WAVES_N
-#undef MLXR_PF_REGBUF
 }  // namespace tile128n
 }  // namespace
 

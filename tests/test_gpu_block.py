@@ -372,11 +372,12 @@ def test_block_residual_and_norm_empty_input(pkg, dev, cfg):
     assert tuple(norm(h).shape) == (0, d)
 
 
-def test_block_token_permutation_equivariance(pkg, dev):
-    """At full c2 size: permuting tokens permutes output rows bit for bit,
-    and repeated runs are bit-identical (size-independent properties)."""
+@pytest.mark.parametrize("T", [64, 160, 224, 600])
+def test_block_token_permutation_equivariance(pkg, dev, T):
+    """At full c2 size, with 8-row work items (T = 64), 16-row ones (10 and 14
+    rows an expert) and M-tiles: permuting tokens permutes output rows bit for
+    bit, and repeated runs are bit-identical (size-independent properties)."""
     bw = weights(pkg, "c2", dev)
-    T = 64
     x = pkg.workloads.make_x(bw.cfg, T, dev, seed=99)
     block = bw.block()
     a = block(x).clone()
@@ -546,10 +547,11 @@ def test_switch_glu_forward_matches_composition(pkg, orc, dev):
 
 @pytest.mark.parametrize("bits", [4, 8])
 def test_switch_glu_tall_prefill_tile(pkg, orc, dev, bits):
-    """The 256-row M-tiles of the prefill GEMMs (taken when the experts
-    average 192 rows or more: here 4096 rows over 16 experts), gated
+    """The 128-row M-tiles of the quantised prefill GEMMs (taken when the
+    experts average more than 64 rows: here 4096 rows over 16 experts), gated
     (gate/up with the SwiGLU epilogue) and down, against the oracle's tiled
-    gather_qmm numerics, one expert much fuller than the rest."""
+    gather_qmm numerics, one expert much fuller than the rest.  (Dense weights'
+    256-row tiles: test_gpu_ops.py, test_dense_tiles.)"""
     W = pkg.workloads
     cfg = W.MoEConfig("tall_tile", d=512, E=16, K=2, f=512, bits=bits, tokens=(2048,))
     bw = W.make_weights(cfg, dev)

@@ -400,6 +400,104 @@ def test_gather_qmm_register_tiles(pkg, dev, bits, N, K, offset, counts):
         assert bool(((got[r, 0].double() - want).abs() <= bound).all())
 
 
+# rows of each expert with 192 and more on average (dense weights: 256-row tiles)
+DENSE_COUNTS = [256, 700, 3, 257, 190, 511, 64, 129]
+
+
+def _ffn_f64(x, ids, gate, up, down, act):
+    """The FFN of dense bf16 experts in 64 bits, with the bf16 values that the
+    activations pass through (gate and up sums, sigmoid, products)."""
+    def rb(v):
+        return v.to(torch.bfloat16).double()
+
+    y = torch.empty((x.shape[0], down.shape[1]), dtype=torch.float64, device=x.device)
+    for e in torch.unique(ids).tolist():
+        r = (ids == e).nonzero()[:, 0]
+        xd = x[r].double()
+        g, u = rb(xd @ gate[e].double().t()), rb(xd @ up[e].double().t())
+        if act == "swiglu":
+            h = rb(g * rb(torch.sigmoid(g)))
+        else:  # the constants as bf16 holds them
+            h = rb(0.5 * g * (1 + torch.tanh(0.796875 * (g + 0.044677734375 * g ** 3))))
+        y[r] = rb(h * u) @ down[e].double().t()
+    return y
+
+
+@pytest.mark.parametrize("counts", [SHORT_COUNTS, TALL_COUNTS], ids=["short", "tall"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("f,d,offset", [
+    (64, 64, 0), (192, 192, 0), (320, 576, 0), (64, 1088, 0), (192, 1152, 0), (320, 512, 1),
+    (64, 2048, 4), (320, 768, 0)])
+def test_gated_register_tiles(pkg, dev, bits, f, d, offset, counts):
+    """The gate/up forms of the register-dequantising tiles: every way their
+    scales load (odd group counts, in vectors, in LDS chunks, `offset` elements
+    off 16-byte alignment; the packed layout's up half starts within the bank)
+    and partial N-tiles.  Equal to the dense FFN of the dequantised weights, and
+    near a 64-bit one that rounds the same activations."""
+    E, B = len(counts), sum(counts)
+    g = torch.Generator(device=dev)
+    g.manual_seed(d + f + bits)
+    ids = torch.repeat_interleave(torch.arange(E, device=dev), torch.tensor(counts, device=dev))
+    ids = ids[torch.randperm(B, generator=g, device=dev)].to(torch.int32)
+    x = torch.randn((B, d), generator=g, device=dev).to(torch.bfloat16)
+
+    def at(v):
+        buf = torch.zeros(v.numel() + offset, dtype=v.dtype, device=dev)
+        buf[offset:] = v.reshape(-1)
+        return buf[offset:].view(v.shape)
+
+    def bank(n, k):
+        w = (torch.randn((E, n, k), generator=g, device=dev) * k ** -0.5).to(torch.bfloat16)
+        q = pkg.ops.quantize(w, 64, bits)
+        return (q[0], at(q[1]), at(q[2])), pkg.ops.dequantize(*q, 64, bits)
+
+    nn = pkg.nn
+    gate, up, down = bank(f, d), bank(f, d), bank(d, f)
+    qs = [nn.QuantizedSwitchLinear(*q, 64, bits) for q, _ in (gate, up, down)]
+    ws = [nn.SwitchLinear(w) for _, w in (gate, up, down)]
+    packed = nn.QuantizedSwitchLinear(
+        *[at(torch.cat((a, b), 1)) if i else torch.cat((a, b), 1)
+          for i, (a, b) in enumerate(zip(gate[0], up[0]))], 64, bits)
+    dense = nn.SwitchLinear(torch.cat((gate[1], up[1]), 1))
+    for act, q, w in (("swiglu", nn.SplitSwitchFfn(*qs), nn.SplitSwitchFfn(*ws)),
+                      ("geglu", nn.PackedSwitchFfn(packed, qs[2], "geglu"),
+                       nn.PackedSwitchFfn(dense, ws[2], "geglu"))):
+        got = q.forward(x, ids[:, None])[:, 0]
+        assert torch.equal(got, w.forward(x, ids[:, None])[:, 0]), act
+        want = _ffn_f64(x, ids, gate[1], up[1], down[1], act)
+        # a bf16 step (2^-8) of the output, and of the few activations whose
+        # f32 and 64-bit values round apart
+        assert float((got.double() - want).norm() / want.norm()) < 4e-3, act
+
+
+@pytest.mark.parametrize("counts", [SHORT_COUNTS, TALL_COUNTS, DENSE_COUNTS],
+                         ids=["64", "128", "256"])
+@pytest.mark.parametrize("f,d", [(64, 64), (320, 576), (192, 512), (128, 2048)])
+def test_dense_tiles(pkg, dev, f, d, counts):
+    """The M-tiles of dense bf16 weights (64, 128 and 256 rows), ragged last
+    tiles among them: one projection within f32 sums and a bf16 rounding of a
+    64-bit product, and the gated FFN near a 64-bit one."""
+    E, B = len(counts), sum(counts)
+    g = torch.Generator(device=dev)
+    g.manual_seed(d + f + B)
+    ids = torch.repeat_interleave(torch.arange(E, device=dev), torch.tensor(counts, device=dev))
+    ids = ids[torch.randperm(B, generator=g, device=dev)].to(torch.int32)
+    x = torch.randn((B, d), generator=g, device=dev).to(torch.bfloat16)
+    gate, up, down = ((torch.randn((E, n, k), generator=g, device=dev) * k ** -0.5)
+                      .to(torch.bfloat16) for n, k in ((f, d), (f, d), (d, f)))
+    got = pkg.ops.gather_mm(x[:, None], gate, None, ids)[:, 0].double()
+    for e in range(E):
+        r = (ids == e).nonzero()[:, 0]
+        xd, wd = x[r].double(), gate[e].double()
+        want = xd @ wd.t()
+        bound = 2.0 ** -8 * want.abs() + d * 2.0 ** -24 * (xd.abs() @ wd.abs().t())
+        assert bool(((got[r] - want).abs() <= bound).all()), e
+    nn = pkg.nn
+    y = nn.SplitSwitchFfn(*map(nn.SwitchLinear, (gate, up, down))).forward(x, ids[:, None])[:, 0]
+    want = _ffn_f64(x, ids, gate, up, down, "swiglu")
+    assert float((y.double() - want).norm() / want.norm()) < 4e-3
+
+
 @pytest.mark.parametrize("counts", [SHORT_COUNTS, TALL_COUNTS], ids=["short", "tall"])
 @pytest.mark.parametrize("f,d,offset", [(64, 512, 0), (320, 768, 0), (128, 2048, 0), (192, 576, 0),
                                         (192, 512, 1)])

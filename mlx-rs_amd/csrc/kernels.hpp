@@ -253,11 +253,13 @@ constexpr int32_t kActGeglu = 1;   // gelu_approx(g) * u  (gemma4 experts)
 // Largest input dim (K) of a projection: 8 waves x 8 groups of 64.
 constexpr int kMaxInputDims = 4096;
 // Prefill kernel M-tiles.  Quantised weights: 64 rows (prefill_reg.hip) while
-// the experts average no more than that, else 128 (prefill_tall.hip); steps
-// with 64- against 128-row tiles: c6 T=2048 (64 rows an expert) 301 us / 310,
-// c5 T=1024 (64) 858 / 891, c2 T=1100 (69) 229 / 199, c2 T=1536 (96) 252 / 233,
-// c3 T=2048 (128) 310 / 289, c3 T=4096 (256) 522 / 467, c7 T=2048 (128)
-// 352 / 361.  Dense bf16 weights: 256 rows when the experts average at least
+// the experts average fewer than that, else 128 (prefill_tall.hip).  Steps with
+// 64- and with 128-row tiles, all from one run: c6 T=1024 (32 rows an expert)
+// 219 us and 224, c5 T=512 (32) 650 and 703, c7 T=512 (32) 183 and 179;
+// c6 T=2048 (64) 298 and 283, c5 T=1024 (64) 838 and 830, c7 T=1024 (64) 233
+// and 218, c2 T=1100 (69) 219 and 190, c2 T=1536 (96) 241 and 213, c3 T=2048
+// (128) 292 and 271, c7 T=2048 (128) 335 and 321, c3 T=4096 (256) 504 and 436.
+// Dense bf16 weights: 256 rows when the experts average at least
 // MLXR_PREFILL_TALL_ROWS rows, 128 from MLXR_PREFILL_DENSE_ROWS (prefill.hip:
 // nothing to keep out of LDS; c8 T=2048 450 us with either height below 256),
 // else 64.  The dispatch cuts its M-tile list with the same choice; tile lists

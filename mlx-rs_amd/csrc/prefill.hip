@@ -62,7 +62,7 @@ namespace tile128n {
 
 int prefill_tile_rows(int64_t rows, int64_t experts, int bits) {
   const int64_t e = experts > 0 ? experts : 1;
-  if (bits != 16) return rows > kPrefillMinTileRows * e ? 128 : kPrefillMinTileRows;
+  if (bits != 16) return rows >= kPrefillMinTileRows * e ? 128 : kPrefillMinTileRows;
   if (rows >= (int64_t)MLXR_PREFILL_TALL_ROWS * e) return tile256::kBM;
   if (rows >= (int64_t)MLXR_PREFILL_DENSE_ROWS * e) return tile128n::kBM;
   return kPrefillMinTileRows;

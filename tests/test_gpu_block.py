@@ -548,7 +548,7 @@ def test_switch_glu_forward_matches_composition(pkg, orc, dev):
 @pytest.mark.parametrize("bits", [4, 8])
 def test_switch_glu_tall_prefill_tile(pkg, orc, dev, bits):
     """The 128-row M-tiles of the quantised prefill GEMMs (taken when the
-    experts average more than 64 rows: here 4096 rows over 16 experts), gated
+    experts average 64 rows or more: here 4096 rows over 16 experts), gated
     (gate/up with the SwiGLU epilogue) and down, against the oracle's tiled
     gather_qmm numerics, one expert much fuller than the rest.  (Dense weights'
     256-row tiles: test_gpu_ops.py, test_dense_tiles.)"""

@@ -351,7 +351,7 @@ def test_gather_lhs_rows_beyond_gathered_count(pkg, orc, dev, bits):
     _close(orc.bf16_to_f32(_np(orc, got)), orc.bf16_to_f32(want), bits)
 
 
-# rows of each expert: up to 64 on average (64-row tiles), and above (128)
+# rows of each expert: below 64 on average (64-row tiles), and above (128)
 SHORT_COUNTS = [64, 1, 32, 33, 65, 31, 0, 63, 2, 17, 96, 48, 30, 34, 5, 20]
 TALL_COUNTS = [300, 1, 127, 128, 129, 96, 97, 65, 33, 0, 64, 200]
 

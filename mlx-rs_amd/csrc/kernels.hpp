@@ -248,6 +248,9 @@ struct QGemmArgs {
 #define MLXR_WIDE_ITEM_ROWS 6
 #endif
 int work_rows_for(int64_t n, int64_t E, std::initializer_list<const QGemmArgs*> gemms);
+inline bool wide_items_possible(int64_t n, int64_t E) {  // by their number alone
+  return n > 64 && n >= MLXR_WIDE_ITEM_ROWS * E;
+}
 constexpr int32_t kActSwiglu = 0;  // silu(g) * u  (Qwen3.5/3.6 experts)
 constexpr int32_t kActGeglu = 1;   // gelu_approx(g) * u  (gemma4 experts)
 // Largest input dim (K) of a projection: 8 waves x 8 groups of 64.

@@ -315,6 +315,7 @@ Status SwitchFfn::forward(const uint16_t* x, int64_t T, const int32_t* indices,
 }
 
 int SwitchFfn::work_rows(int64_t n, const SharedFold* fold) const {
+  if (!wide_items_possible(n, sw_.E)) return kWorkRows;
   const QGemmArgs g = gemm_shape(sw_.gate, sw_.up, true, sw_.f, sw_.d, sw_.bits);
   const QGemmArgs h = gemm_shape(sw_.down, QWeights{}, false, sw_.d, sw_.f, sw_.bits);
   if (!fold) return work_rows_for(n, sw_.E, {&g, &h});

@@ -156,6 +156,7 @@ __device__ __forceinline__ void decode_body(const QGemmArgs& a, int tile,
   constexpr int GPS = BITS == 4 ? 2 : 1;
   constexpr int GW = SPW * GPS;          // groups per wave per pass
   constexpr int NX = BITS == 4 ? 4 : 2;  // x fragments per step
+  constexpr bool kWide = BITS != 16;     // items of over kWorkRows rows, too
   const int kw = blockDim.x >> 6;
   const int e = wk.x, row0 = wk.y, rows = wk.z;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -175,11 +176,12 @@ __device__ __forceinline__ void decode_body(const QGemmArgs& a, int tile,
     int64_t xrow = 0;
     if (tv) {
       const int slot = row0 + tok;
-      // this lane's flat row from the record (its first eight fetched with the
-      // header; a wide item's others from the sorted list)
+      // this lane's flat row from the record (its eight fetched with the header;
+      // a wide item's others from the sorted list)
       const int f4 = (tok & 3) == 0 ? fr0.x : (tok & 3) == 1 ? fr0.y : (tok & 3) == 2 ? fr0.z : fr0.w;
       const int f8 = (tok & 3) == 0 ? fr1.x : (tok & 3) == 1 ? fr1.y : (tok & 3) == 2 ? fr1.z : fr1.w;
-      const int flat = tok < 4 ? f4 : tok < kWorkRows ? f8 : a.x_by_slot ? 0 : a.sorted[slot];
+      int flat = tok < 4 ? f4 : f8;
+      if (kWide && tok >= kWorkRows && !a.x_by_slot) flat = a.sorted[slot];
       xrow = a.x_by_slot ? slot : (a.row_map ? a.row_map[flat] : flat / a.row_div);
     }
     f32x4_t acc[CB][NM];
@@ -316,8 +318,8 @@ __device__ __forceinline__ void decode_body(const QGemmArgs& a, int tile,
             a.out[(int64_t)slot * a.out_ld + ch] =
                 gated_act_bf16(a.act, bf16_round(s0[r]), bf16_round(s1[r]));
           } else {
-            const int64_t orow =
-                !a.out_by_flat ? slot : t < kWorkRows ? rec[4 + t] : a.sorted[slot];
+            int64_t orow = slot;
+            if (a.out_by_flat) orow = !kWide || t < kWorkRows ? rec[4 + t] : a.sorted[slot];
             a.out[orow * a.out_ld + ch] = f32_to_bf16(s0[r]);
           }
         }
@@ -331,7 +333,7 @@ template <int BITS, bool GATED, int SPW, int CB>
 __global__ __launch_bounds__(1024) void qgemm_decode_kernel(
     QGemmArgs a, int tiles_n, QGemmArgs a2, int units1, int items1, int rows2) {
   Unit u;
-  if (!decode_unit<0>(a, tiles_n, units1, items1, rows2, u)) return;
+  if (!decode_unit<BITS == 16 ? kWorkRows : 0>(a, tiles_n, units1, items1, rows2, u)) return;
   decode_body<BITS, GATED, SPW, CB>(u.shared ? a2 : a, u.tile, u.rec, u.wk,
                                     u.fr0, u.fr1);
 }
@@ -528,7 +530,7 @@ StreamShape stream_shape(const QGemmArgs& a, int64_t all_items) {
 }  // namespace
 
 int work_rows_for(int64_t n, int64_t E, std::initializer_list<const QGemmArgs*> gemms) {
-  if (n <= 64 || n < MLXR_WIDE_ITEM_ROWS * E) return kWorkRows;
+  if (!wide_items_possible(n, E)) return kWorkRows;
   const int64_t items = dispatch_max_work(n, E, kWorkRowsWide);
   for (const QGemmArgs* g : gemms) {
     if (g->bits == 16 || !(g->K <= kWideWhole || g->K % kWideSlice == 0) ||

@@ -16,12 +16,13 @@
 // ahead, a barrier per group, two workgroups per CU.
 //
 // c3 T=4096 (256 rows an expert on average, skewed) against 256 x 256 tiles
-// through LDS: gate/up 264 to 253 us, down 164 to 136, step 499 to 466; a copy
-// that only reads x and multiplies takes 174 us for gate/up.  The matrix cores
-// are busy 40% of the launch, they or the VALU 62%.  No faster: the MFMAs of a
-// chunk kept together, raised wave priority around them (step 519), one MFMA
-// to every 4 or 5 VALU instructions by scheduling groups (489, 505), the order
-// pinned instruction group by instruction group (475).
+// through LDS, both from one run: step 509 to 446 us; first passes on new
+// inputs, traced, gate/up 288 to 242, down 176 to 134.  A copy that only reads x
+// and multiplies takes 174 us for gate/up.  The matrix cores
+// are busy 39% of it, 35% of down.  No faster, against a step of 466 us then:
+// the MFMAs of a chunk kept together, raised wave priority around them (519),
+// one MFMA to every 4 or 5 VALU instructions by scheduling groups (489, 505),
+// the order pinned instruction group by instruction group (475).
 #include <algorithm>
 
 #include "common.hpp"

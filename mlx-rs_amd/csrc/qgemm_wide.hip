@@ -26,8 +26,11 @@ namespace {
 // quarter by quarter, so MFMA i here is MFMAs 2 i and 2 i + 1 there, and the
 // groups A and the groups B are summed apart (acc[0], acc[1]) and joined at a
 // block's end, as its two halves of the wave are.  x is staged whole up
-// to kWideWhole inputs, else kWideSlice at a time (so that three workgroups
-// still share a CU), NB = 1 then.
+// to kWideWhole inputs, else kWideSlice at a time, NB = 1 then: three
+// workgroups share a CU up to K = 2048 (above, the 8-token form, which stages
+// all of K, and the scales leave room for two at K = 3072 and for one at 4096).
+// The gated 4-bit kernel keeps one register pair in scratch across its 4-token
+// loop; no loop reads it.
 // 12 rows an expert of c7 (T = 190): gate/up 83 us in 8-row items, 72 in these,
 // down 59 and 44.  Steps of c2 at 8, 10 and 14 rows an expert (T = 128, 160,
 // 224): 128, 151, 186 us and 117, 130, 154; c5 at 6 (T = 200) 893 and 810.
